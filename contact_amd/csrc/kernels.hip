@@ -53,8 +53,46 @@ __device__ inline double combine(double a, double b, int mode)
     return mode == 0 ? a + b : (mode == 1 ? fmax(a, b) : fmin(a, b));
 }
 
-// work-group reduction of K values; result valid in thread 0.  Wave-level steps use
-// cross-lane shuffles (DPP on CDNA), then one LDS exchange between the waves.
+// Cross-lane moves of the wave reductions, on the VALU (DPP and the half swaps of CDNA4) where
+// __shfl_xor goes through the LDS pipe: 64-bit values as two 32-bit halves.
+template <int CTRL>
+__device__ inline double dpp_f64(double v)
+{
+    const int lo = __builtin_amdgcn_update_dpp(0, __double2loint(v), CTRL, 0xF, 0xF, false);
+    const int hi = __builtin_amdgcn_update_dpp(0, __double2hiint(v), CTRL, 0xF, 0xF, false);
+    return __hiloint2double(hi, lo);
+}
+// v of lane ^ 32 and of lane ^ 16
+__device__ inline double xor32_f64(double v)
+{
+    const auto l = __builtin_amdgcn_permlane32_swap(__double2loint(v), __double2loint(v), false, false);
+    const auto h = __builtin_amdgcn_permlane32_swap(__double2hiint(v), __double2hiint(v), false, false);
+    const bool up = threadIdx.x & 32;
+    return __hiloint2double(up ? h[0] : h[1], up ? l[0] : l[1]);
+}
+__device__ inline double xor16_f64(double v)
+{
+    const auto l = __builtin_amdgcn_permlane16_swap(__double2loint(v), __double2loint(v), false, false);
+    const auto h = __builtin_amdgcn_permlane16_swap(__double2hiint(v), __double2hiint(v), false, false);
+    const bool up = threadIdx.x & 16;
+    return __hiloint2double(up ? h[0] : h[1], up ? l[0] : l[1]);
+}
+// The butterfly over lane ^ 32, 16, 8, 4, 2, 1, in that order.  After the first three steps a
+// value depends on its lane mod 8 only, so that a rotation by 4 within 16 lanes brings the
+// value of lane ^ 4.  Every lane ends with the same bits as a butterfly of __shfl_xor gives.
+// Needs all 64 lanes of the wave.
+__device__ inline double wave_combine(double x, int mode)
+{
+    x = combine(x, xor32_f64(x), mode);
+    x = combine(x, xor16_f64(x), mode);
+    x = combine(x, dpp_f64<0x128>(x), mode);   // row_ror:8
+    x = combine(x, dpp_f64<0x124>(x), mode);   // row_ror:4
+    x = combine(x, dpp_f64<0x4E>(x), mode);    // quad_perm [2,3,0,1]
+    return combine(x, dpp_f64<0xB1>(x), mode); // quad_perm [1,0,3,2]
+}
+
+// work-group reduction of K values; result valid in thread 0.  Wave-level steps on the VALU,
+// then one LDS exchange between the waves.
 template <int K>
 __device__ inline void group_reduce(double (&v)[K], int mode, double* lds)
 {
@@ -62,11 +100,7 @@ __device__ inline void group_reduce(double (&v)[K], int mode, double* lds)
     const int wave = threadIdx.x >> 6;
     const int nwave = (blockDim.x + 63) >> 6;
 #pragma unroll
-    for (int k = 0; k < K; k++) {
-        double x = v[k];
-        for (int off = 32; off > 0; off >>= 1) x = combine(x, __shfl_xor(x, off), mode);
-        v[k] = x;
-    }
+    for (int k = 0; k < K; k++) v[k] = wave_combine(v[k], mode);
     __syncthreads();
     if (lane == 0)
         for (int k = 0; k < K; k++) lds[wave * K + k] = v[k];
@@ -85,58 +119,87 @@ __device__ inline double combine_identity(int mode)
     return mode == 0 ? 0.0 : (mode == 1 ? -INFINITY : INFINITY);
 }
 
-// The last work-group of an item to finish combines the item's group partials: one wave, lane
-// l taking groups l, l + 64, ... in order, then a butterfly over the lanes -- a fixed order
-// that depends only on the item's group count, so an item's result is the same whichever
-// other items share the launch.
-template <int K>
-__device__ inline void final_reduce(const RedOut& ro, const int* gstart, int it, double* extra = nullptr)
-{
-    __threadfence();   // acquire: the other groups' partials
-    if (threadIdx.x >= 64) return;
-    const int lane = threadIdx.x, g0 = gstart[it], g1 = gstart[it + 1];
-    const int mode = ro.modes[it];
-    for (int k = 0; k < K; k++) {
-        double x = combine_identity(mode);
-        for (int g = g0 + lane; g < g1; g += 64) x = combine(x, ro.partials[(size_t)g * K + k], mode);
-        for (int off = 32; off > 0; off >>= 1) x = combine(x, __shfl_xor(x, off), mode);
-        if (lane == 0) {
-            ro.results[(size_t)it * K + k] = x;
-            if (extra) extra[k] = x;   // the item's device copy, read by later launches
-        }
-    }
-    if (lane == 0) ro.count[it] = 0u;   // ready for the next launch that uses this counter
-}
-
 // Reduce K values over the work-group and store the group's partials; with ro.count set, the
-// item's last group also forms the item's results (no separate finalize launch).  Must be
-// reached by every thread of the group.
+// item's last group to arrive also forms the item's results (no separate finalize launch): one
+// wave, lane l taking the partials of groups l, l + 64, ... in order, then a butterfly over the
+// lanes -- an order that depends only on the item's group count, so an item's result is the same
+// whichever other items share the launch.  `extra` receives a copy that later launches read.
+// Must be reached by every thread of the group.
+//
+// What a reduction adds to a launch is latency.  An item of one group (up to 1024 elements)
+// needs no arrival at all.  With several groups, only the partials pass between groups: they
+// are stored and loaded as agent-scope atomics (past the caches of the XCD), and the group waits
+// for its stores before it arrives.  A fence would first write the XCD's L2 back, the vectors
+// that the kernel has just stored included.  Measured (k_vec, average over its operations of a
+// solve, HIP events of about 4 us included): 42.0 us a launch with fences and LDS shuffles, 18.4
+// us so for one 1024 x 1024 patch (1024 groups), 18.9 and 9.8 us for 512 x 512, 12.5 and 7.1 us
+// for 40 x 40.
 template <int K>
 __device__ inline void write_partials(double (&v)[K], int mode, const RedOut& ro, const int* gstart, int it,
                                       double* extra = nullptr)
 {
     __shared__ double red_lds[16 * MAXK];
-    __shared__ int s_last;
-    group_reduce<K>(v, mode, red_lds);
-    if (threadIdx.x == 0) {
-        for (int k = 0; k < K; k++) ro.partials[(size_t)blockIdx.x * K + k] = v[k];
-        int last = 0;
-        if (ro.count) {
-            __threadfence();   // release: this group's partials before its arrival
-            const unsigned ng = (unsigned)(gstart[it + 1] - gstart[it]);
-            last = atomicAdd(&ro.count[it], 1u) == ng - 1u;
-        }
-        s_last = last;
-    }
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, nwave = (blockDim.x + 63) >> 6;
+#pragma unroll
+    for (int k = 0; k < K; k++) v[k] = wave_combine(v[k], mode);
     __syncthreads();
-    if (s_last) final_reduce<K>(ro, gstart, it, extra);
+    if (lane == 0)
+        for (int k = 0; k < K; k++) red_lds[wave * K + k] = v[k];
+    __syncthreads();
+    if (wave != 0) return;
+    const int g0 = gstart[it], g1 = gstart[it + 1];
+    // lane k: the group's value k, the waves in order
+    double x = 0.0;
+    if (lane < K) {
+        x = red_lds[lane];
+        for (int w = 1; w < nwave; w++) x = combine(x, red_lds[w * K + lane], mode);
+    }
+    if (!ro.count) {
+        if (lane < K) ro.partials[(size_t)blockIdx.x * K + lane] = x;
+        return;
+    }
+    if (g1 - g0 == 1) {
+        if (lane < K) {
+            x = combine(combine_identity(mode), x, mode);
+            ro.results[(size_t)it * K + lane] = x;
+            if (extra) extra[lane] = x;
+        }
+        return;
+    }
+    if (lane < K)
+        __hip_atomic_store(&ro.partials[(size_t)blockIdx.x * K + lane], x, __ATOMIC_RELAXED,
+                           __HIP_MEMORY_SCOPE_AGENT);
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    unsigned arrived = 0;
+    if (lane == 0)
+        arrived = __hip_atomic_fetch_add(&ro.count[it], 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    arrived = __builtin_amdgcn_readfirstlane(arrived);
+    if (arrived != (unsigned)(g1 - g0) - 1u) return;
+    asm volatile("" ::: "memory");
+    double y[K];
+#pragma unroll
+    for (int k = 0; k < K; k++) y[k] = combine_identity(mode);
+    for (int g = g0 + lane; g < g1; g += 64)
+#pragma unroll
+        for (int k = 0; k < K; k++)
+            y[k] = combine(y[k], __hip_atomic_load(&ro.partials[(size_t)g * K + k], __ATOMIC_RELAXED,
+                                                   __HIP_MEMORY_SCOPE_AGENT), mode);
+#pragma unroll
+    for (int k = 0; k < K; k++) {
+        const double r = wave_combine(y[k], mode);
+        if (lane == 0) {
+            ro.results[(size_t)it * K + k] = r;
+            if (extra) extra[k] = r;
+        }
+    }
+    if (lane == 0) ro.count[it] = 0u;   // ready for the next launch that uses this counter
 }
 
 // ------------------------------------------------------------------------------------------
 // masked BLAS-1 (src/m_gridfunc.f90:936-1650)
 // ------------------------------------------------------------------------------------------
 
-__global__ void __launch_bounds__(ELEM_THREADS) k_vec(const VecItem* items, const int* gstart,
+__global__ void __launch_bounds__(ELEM_THREADS) k_vec(const VecItem* __restrict__ items, const int* __restrict__ gstart,
                                                       int nitems, RedOut ro)
 {
     int it = find_item(gstart, nitems, blockIdx.x);
@@ -163,28 +226,74 @@ __global__ void __launch_bounds__(ELEM_THREADS) k_vec(const VecItem* items, cons
         if (fabs(vav) > 1e-32 && I.flag) a = rv / vav;
         else a = rv / fmax(NCG_TINY, vav);
     }
+    // the thread's elements, then per operation all loads before the arithmetic
+    const int n = I.n, ncomp = I.ncomp, mask = I.mask;
+    const int8_t* const el = I.el;
+    int idx[ELEM_PER_THREAD];
+    bool on[ELEM_PER_THREAD];
+#pragma unroll
     for (int e = 0; e < ELEM_PER_THREAD; e++) {
-        int i = base + e * ELEM_THREADS + threadIdx.x;
-        if (i >= I.n) break;
-        if (!in_mask(I.mask, I.el ? I.el[i] : (int8_t)0)) continue;
-        for (int c = 0; c < I.ncomp; c++) {
+        idx[e] = base + e * ELEM_THREADS + threadIdx.x;
+        on[e] = idx[e] < n;
+    }
+    if (mask != M_ALL) {
+        int8_t st[ELEM_PER_THREAD];
+#pragma unroll
+        for (int e = 0; e < ELEM_PER_THREAD; e++) st[e] = on[e] && el ? el[idx[e]] : (int8_t)0;
+#pragma unroll
+        for (int e = 0; e < ELEM_PER_THREAD; e++) on[e] = on[e] && in_mask(mask, st[e]);
+    }
+    if (sub <= V_ADDC) {
+        // updates: nothing to reduce
+        for (int c = 0; c < ncomp; c++) {
+            double* const x = I.x[c];
+            double* const y = I.y[c];
+            double vx[ELEM_PER_THREAD], vy[ELEM_PER_THREAD];
+            const bool rx = sub != V_SET, ry = sub == V_AXPY || sub == V_AXPBY;
+#pragma unroll
+            for (int e = 0; e < ELEM_PER_THREAD; e++) {
+                vx[e] = rx && on[e] ? x[idx[e]] : 0.0;
+                vy[e] = ry && on[e] ? y[idx[e]] : 0.0;
+            }
+            double* const dst = sub == V_COPY || ry ? y : x;
+#pragma unroll
+            for (int e = 0; e < ELEM_PER_THREAD; e++) {
+                double r = a;                                  // V_SET
+                if (sub == V_COPY) r = vx[e];
+                else if (sub == V_SCAL) r = vx[e] * a;
+                else if (sub == V_AXPY) r = vy[e] + a * vx[e];
+                else if (sub == V_AXPBY) r = a * vx[e] + b * vy[e];
+                else if (sub == V_ADDC) r = vx[e] + a;
+                if (on[e]) dst[idx[e]] = r;
+            }
+        }
+        return;
+    }
+    double vx[2][ELEM_PER_THREAD], vy[2][ELEM_PER_THREAD];
+#pragma unroll
+    for (int c = 0; c < 2; c++)
+#pragma unroll
+        for (int e = 0; e < ELEM_PER_THREAD; e++) {
+            const bool rd = c < ncomp && on[e] && sub != V_COUNT;
+            vx[c][e] = rd ? I.x[c][idx[e]] : 0.0;
+            vy[c][e] = rd && sub == V_DOT ? I.y[c][idx[e]] : 0.0;
+        }
+#pragma unroll
+    for (int e = 0; e < ELEM_PER_THREAD; e++)
+#pragma unroll
+        for (int c = 0; c < 2; c++) {
+            if (!on[e] || c >= ncomp) continue;
+            const double x = vx[c][e];
             switch (sub) {
-            case V_SET: I.x[c][i] = a; break;
-            case V_COPY: I.y[c][i] = I.x[c][i]; break;
-            case V_SCAL: I.x[c][i] *= a; break;
-            case V_AXPY: I.y[c][i] += a * I.x[c][i]; break;
-            case V_AXPBY: I.y[c][i] = a * I.x[c][i] + b * I.y[c][i]; break;
-            case V_ADDC: I.x[c][i] += a; break;
-            case V_DOT: acc[0] += I.x[c][i] * I.y[c][i]; acc[1] += 1.0; break;
-            case V_SUM: acc[0] += I.x[c][i]; acc[1] += 1.0; break;
-            case V_SUMSQ: acc[0] += I.x[c][i] * I.x[c][i]; acc[1] += 1.0; break;
-            case V_MAXABS: acc[0] = fmax(acc[0], fabs(I.x[c][i])); break;
-            case V_MIN: acc[0] = fmin(acc[0], I.x[c][i]); break;
-            case V_MAX: acc[0] = fmax(acc[0], I.x[c][i]); break;
+            case V_DOT: acc[0] += x * vy[c][e]; acc[1] += 1.0; break;
+            case V_SUM: acc[0] += x; acc[1] += 1.0; break;
+            case V_SUMSQ: acc[0] += x * x; acc[1] += 1.0; break;
+            case V_MAXABS: acc[0] = fmax(acc[0], fabs(x)); break;
+            case V_MIN: acc[0] = fmin(acc[0], x); break;
+            case V_MAX: acc[0] = fmax(acc[0], x); break;
             case V_COUNT: acc[0] += 1.0; break;
             }
         }
-    }
     // max/min: the second value is 0 (the count of the sums); the group reduction of
     // zeros under max or min stays 0.  The echoed scalars enter the sums once, from the
     // item's first group's first thread.
@@ -202,7 +311,7 @@ __global__ void __launch_bounds__(ELEM_THREADS) k_vec(const VecItem* items, cons
 
 // interior elements with negative pressure move to the exterior (src/m_solvpn.f90:302-311);
 // returns (#moved, #interior after, sum pn)
-__global__ void __launch_bounds__(ELEM_THREADS) k_ncg_negpn(const NcgItem* items, const int* gstart,
+__global__ void __launch_bounds__(ELEM_THREADS) k_ncg_negpn(const NcgItem* __restrict__ items, const int* __restrict__ gstart,
                                                             int nitems, RedOut ro)
 {
     int it = find_item(gstart, nitems, blockIdx.x);
@@ -227,7 +336,7 @@ __global__ void __launch_bounds__(ELEM_THREADS) k_ncg_negpn(const NcgItem* items
 
 // elements at the deepest interpenetration enter: mode 1 at the start of NormCG with N=1
 // (src/m_solvpn.f90:140-152), mode 2 when no contact is left (src/m_solvpn.f90:316-326)
-__global__ void __launch_bounds__(ELEM_THREADS) k_ncg_hmin(const NcgItem* items, const int* gstart,
+__global__ void __launch_bounds__(ELEM_THREADS) k_ncg_hmin(const NcgItem* __restrict__ items, const int* __restrict__ gstart,
                                                            int nitems, RedOut ro)
 {
     int it = find_item(gstart, nitems, blockIdx.x);
@@ -248,7 +357,7 @@ __global__ void __launch_bounds__(ELEM_THREADS) k_ncg_hmin(const NcgItem* items,
 }
 
 // dd = A ps - rhs on all elements; returns (sum dd, count) over the interior
-__global__ void __launch_bounds__(ELEM_THREADS) k_ncg_dd(const NcgItem* items, const int* gstart,
+__global__ void __launch_bounds__(ELEM_THREADS) k_ncg_dd(const NcgItem* __restrict__ items, const int* __restrict__ gstart,
                                                          int nitems, RedOut ro)
 {
     int it = find_item(gstart, nitems, blockIdx.x);
@@ -267,7 +376,7 @@ __global__ void __launch_bounds__(ELEM_THREADS) k_ncg_dd(const NcgItem* items, c
 
 // proj_avg of dd, residual, and interpenetration check of the exterior
 // (src/m_solvpn.f90:351-390); returns #elements that entered
-__global__ void __launch_bounds__(ELEM_THREADS) k_ncg_expand(const NcgItem* items, const int* gstart,
+__global__ void __launch_bounds__(ELEM_THREADS) k_ncg_expand(const NcgItem* __restrict__ items, const int* __restrict__ gstart,
                                                              int nitems, RedOut ro)
 {
     int it = find_item(gstart, nitems, blockIdx.x);
@@ -298,7 +407,7 @@ __global__ void __launch_bounds__(ELEM_THREADS) k_ncg_expand(const NcgItem* item
 }
 
 // snorm contract step (src/m_snorm.f90:196-219): returns (#moved out, #small pn)
-__global__ void __launch_bounds__(ELEM_THREADS) k_sn_contract(const NcgItem* items, const int* gstart,
+__global__ void __launch_bounds__(ELEM_THREADS) k_sn_contract(const NcgItem* __restrict__ items, const int* __restrict__ gstart,
                                                               int nitems, RedOut ro)
 {
     int it = find_item(gstart, nitems, blockIdx.x);
@@ -321,7 +430,7 @@ __global__ void __launch_bounds__(ELEM_THREADS) k_sn_contract(const NcgItem* ite
 }
 
 // snorm expand step (src/m_snorm.f90:253-286): returns (#moved in, #small dd)
-__global__ void __launch_bounds__(ELEM_THREADS) k_sn_expand(const NcgItem* items, const int* gstart,
+__global__ void __launch_bounds__(ELEM_THREADS) k_sn_expand(const NcgItem* __restrict__ items, const int* __restrict__ gstart,
                                                             int nitems, RedOut ro)
 {
     int it = find_item(gstart, nitems, blockIdx.x);
@@ -344,7 +453,7 @@ __global__ void __launch_bounds__(ELEM_THREADS) k_sn_expand(const NcgItem* items
 }
 
 // final regularisation (src/m_snorm.f90:315-325)
-__global__ void __launch_bounds__(ELEM_THREADS) k_sn_final(const NcgItem* items, const int* gstart,
+__global__ void __launch_bounds__(ELEM_THREADS) k_sn_final(const NcgItem* __restrict__ items, const int* __restrict__ gstart,
                                                            int nitems, RedOut ro)
 {
     int it = find_item(gstart, nitems, blockIdx.x);
@@ -366,7 +475,7 @@ __global__ void __launch_bounds__(ELEM_THREADS) k_sn_final(const NcgItem* items,
 // gf3_AijPj with unit tractions at one element: sum over rows jy of the coefficients for
 // jx in [row1st-1, rowlst+1] of the current contact area (src/m_aijpj.f90:158-185,
 // src/m_gridfunc.f90:582-637).  One group per item, one thread per row.
-__global__ void __launch_bounds__(ROW_THREADS) k_aij_ones(const AijItem* items, const int* gstart,
+__global__ void __launch_bounds__(ROW_THREADS) k_aij_ones(const AijItem* __restrict__ items, const int* __restrict__ gstart,
                                                           int nitems, RedOut ro)
 {
     int it = find_item(gstart, nitems, blockIdx.x);
@@ -406,7 +515,7 @@ __device__ inline void nt_from_p(double px, double py, double& nx, double& ny)
     ny = sin(th);
 }
 
-__global__ void __launch_bounds__(ELEM_THREADS) k_tcg_nt(const TcgItem* items, const int* gstart,
+__global__ void __launch_bounds__(ELEM_THREADS) k_tcg_nt(const TcgItem* __restrict__ items, const int* __restrict__ gstart,
                                                          int nitems, RedOut ro)
 {
     int it = find_item(gstart, nitems, blockIdx.x);
@@ -423,7 +532,7 @@ __global__ void __launch_bounds__(ELEM_THREADS) k_tcg_nt(const TcgItem* items, c
 }
 
 // r = -s, projected on t in the slip area
-__global__ void __launch_bounds__(ELEM_THREADS) k_tcg_rset(const TcgItem* items, const int* gstart,
+__global__ void __launch_bounds__(ELEM_THREADS) k_tcg_rset(const TcgItem* __restrict__ items, const int* __restrict__ gstart,
                                                            int nitems, RedOut ro)
 {
     int it = find_item(gstart, nitems, blockIdx.x);
@@ -445,7 +554,7 @@ __global__ void __launch_bounds__(ELEM_THREADS) k_tcg_rset(const TcgItem* items,
 }
 
 // Jacobian diagonal scaling and slip projection of z; returns (z.q, v.q) over all elements
-__global__ void __launch_bounds__(ELEM_THREADS) k_tcg_zprep(const TcgItem* items, const int* gstart,
+__global__ void __launch_bounds__(ELEM_THREADS) k_tcg_zprep(const TcgItem* __restrict__ items, const int* __restrict__ gstart,
                                                             int nitems, RedOut ro)
 {
     int it = find_item(gstart, nitems, blockIdx.x);
@@ -478,7 +587,7 @@ __global__ void __launch_bounds__(ELEM_THREADS) k_tcg_zprep(const TcgItem* items
 }
 
 // v = z + beta v with beta from zprep's (z.q, v.q) in sc[0..1] (src/m_solvpt.f90:2150-2160)
-__global__ void __launch_bounds__(ELEM_THREADS) k_tcg_vupd(const TcgItem* items, const int* gstart,
+__global__ void __launch_bounds__(ELEM_THREADS) k_tcg_vupd(const TcgItem* __restrict__ items, const int* __restrict__ gstart,
                                                            int nitems, RedOut ro)
 {
     int it = find_item(gstart, nitems, blockIdx.x);
@@ -498,7 +607,7 @@ __global__ void __launch_bounds__(ELEM_THREADS) k_tcg_vupd(const TcgItem* items,
 }
 
 // q: slip projection and curvature term; returns (r.v, v.q)
-__global__ void __launch_bounds__(ELEM_THREADS) k_tcg_qpost(const TcgItem* items, const int* gstart,
+__global__ void __launch_bounds__(ELEM_THREADS) k_tcg_qpost(const TcgItem* __restrict__ items, const int* __restrict__ gstart,
                                                             int nitems, RedOut ro)
 {
     int it = find_item(gstart, nitems, blockIdx.x);
@@ -530,7 +639,7 @@ __global__ void __launch_bounds__(ELEM_THREADS) k_tcg_qpost(const TcgItem* items
 // pold = p; p += alpha v (interior); slip clipped to the bound; returns (sum v^2, sum p^2), or
 // sum (p - p0)^2 in a sensitivity solve (src/m_solvpt.f90:2209-2216), then (r.v, v.q).  With
 // sc set, alpha is formed here from qpost's (r.v, v.q) in sc[2..3] (:2190-2200).
-__global__ void __launch_bounds__(ELEM_THREADS) k_tcg_pupd(const TcgItem* items, const int* gstart,
+__global__ void __launch_bounds__(ELEM_THREADS) k_tcg_pupd(const TcgItem* __restrict__ items, const int* __restrict__ gstart,
                                                            int nitems, RedOut ro)
 {
     int it = find_item(gstart, nitems, blockIdx.x);
@@ -578,7 +687,7 @@ __global__ void __launch_bounds__(ELEM_THREADS) k_tcg_pupd(const TcgItem* items,
 }
 
 // adhesion elements above the traction bound move to slip; returns #moved
-__global__ void __launch_bounds__(ELEM_THREADS) k_tcg_as(const TcgItem* items, const int* gstart,
+__global__ void __launch_bounds__(ELEM_THREADS) k_tcg_as(const TcgItem* __restrict__ items, const int* __restrict__ gstart,
                                                          int nitems, RedOut ro)
 {
     int it = find_item(gstart, nitems, blockIdx.x);
@@ -604,7 +713,7 @@ __global__ void __launch_bounds__(ELEM_THREADS) k_tcg_as(const TcgItem* items, c
 }
 
 // slip elements with s.p > 0 move to adhesion; pold -= p; returns (#moved, sum (pold-p)^2)
-__global__ void __launch_bounds__(ELEM_THREADS) k_tcg_sa(const TcgItem* items, const int* gstart,
+__global__ void __launch_bounds__(ELEM_THREADS) k_tcg_sa(const TcgItem* __restrict__ items, const int* __restrict__ gstart,
                                                          int nitems, RedOut ro)
 {
     int it = find_item(gstart, nitems, blockIdx.x);
@@ -633,7 +742,7 @@ __global__ void __launch_bounds__(ELEM_THREADS) k_tcg_sa(const TcgItem* items, c
 // stang outer loop moves (src/m_stang.f90:433-508)
 // ------------------------------------------------------------------------------------------
 
-__global__ void __launch_bounds__(ELEM_THREADS) k_st_as(const StItem* items, const int* gstart,
+__global__ void __launch_bounds__(ELEM_THREADS) k_st_as(const StItem* __restrict__ items, const int* __restrict__ gstart,
                                                         int nitems, RedOut ro)
 {
     int it = find_item(gstart, nitems, blockIdx.x);
@@ -658,7 +767,7 @@ __global__ void __launch_bounds__(ELEM_THREADS) k_st_as(const StItem* items, con
     write_partials<1>(acc, 0, ro, gstart, it);
 }
 
-__global__ void __launch_bounds__(ELEM_THREADS) k_st_sa(const StItem* items, const int* gstart,
+__global__ void __launch_bounds__(ELEM_THREADS) k_st_sa(const StItem* __restrict__ items, const int* __restrict__ gstart,
                                                         int nitems, RedOut ro)
 {
     int it = find_item(gstart, nitems, blockIdx.x);
@@ -703,7 +812,7 @@ __host__ __device__ inline int gd_rows_per_tile(int mx, int my, int tile)
 __host__ __device__ inline int gd_row_stride(int mx) { return mx | 1; }
 
 // compute_dp, src/gdsteady.f90:610-635: dp = backward differences along x (element-wise)
-__global__ void __launch_bounds__(ELEM_THREADS) k_gd_dp(const GdItem* items, const int* gstart,
+__global__ void __launch_bounds__(ELEM_THREADS) k_gd_dp(const GdItem* __restrict__ items, const int* __restrict__ gstart,
                                                         int nitems, RedOut ro)
 {
     int it = find_item(gstart, nitems, blockIdx.x);
@@ -724,7 +833,7 @@ __global__ void __launch_bounds__(ELEM_THREADS) k_gd_dp(const GdItem* items, con
 }
 
 // project_searchdir, src/gdsteady.f90:639-803: dv from the residual r, with v // t in slip
-__global__ void __launch_bounds__(GD_THREADS) k_gd_project(const GdItem* items, const int* gstart,
+__global__ void __launch_bounds__(GD_THREADS) k_gd_project(const GdItem* __restrict__ items, const int* __restrict__ gstart,
                                                            int nitems, RedOut ro)
 {
     extern __shared__ double gd_lds[];
@@ -834,7 +943,7 @@ __global__ void __launch_bounds__(GD_THREADS) k_gd_project(const GdItem* items, 
 // dp + alpha dv, then the residual terms of the new orientation.  Returns
 // (rho, c0adh, c1adh, c0slp, c1slp, c2slp) and, when I.first, also
 // (sum r^2, sum r.q dscl, sum_int (dscl q)^2, sum_int r^2).
-__global__ void __launch_bounds__(GD_THREADS) k_gd_probe(const GdItem* items, const int* gstart,
+__global__ void __launch_bounds__(GD_THREADS) k_gd_probe(const GdItem* __restrict__ items, const int* __restrict__ gstart,
                                                          int nitems, RedOut ro)
 {
     extern __shared__ double gd_lds[];
@@ -938,7 +1047,7 @@ __global__ void __launch_bounds__(GD_THREADS) k_gd_probe(const GdItem* items, co
 }
 
 // pold = p; dp += alpha dv on the interior; apply_trcbnd (src/gdsteady.f90:807-847); n from p
-__global__ void __launch_bounds__(GD_THREADS) k_gd_update(const GdItem* items, const int* gstart,
+__global__ void __launch_bounds__(GD_THREADS) k_gd_update(const GdItem* __restrict__ items, const int* __restrict__ gstart,
                                                           int nitems, RedOut ro)
 {
     extern __shared__ double gd_lds[];
@@ -1195,7 +1304,7 @@ __device__ void elmtrc(int8_t& el, const double c11, const double c12, const dou
 }
 
 // element-state moves after a GD step (src/gdsteady.f90:375-418); returns #changes
-__global__ void __launch_bounds__(ELEM_THREADS) k_gd_moves(const GdItem* items, const int* gstart,
+__global__ void __launch_bounds__(ELEM_THREADS) k_gd_moves(const GdItem* __restrict__ items, const int* __restrict__ gstart,
                                                            int nitems, RedOut ro)
 {
     int it = find_item(gstart, nitems, blockIdx.x);
@@ -1266,7 +1375,7 @@ __device__ inline bool gd_slip_split(const GdItem& I, int ii, int8_t& elnew, dou
 
 // compute_diagscaling and the scaled residual (src/gdsteady.f90:901-1042, 429-439); when
 // not I.first also pold -= p on the interior.  Returns (sum (pold)^2, sum p^2, sum_int r^2).
-__global__ void __launch_bounds__(ELEM_THREADS) k_gd_diagres(const GdItem* items, const int* gstart,
+__global__ void __launch_bounds__(ELEM_THREADS) k_gd_diagres(const GdItem* __restrict__ items, const int* __restrict__ gstart,
                                                              int nitems, RedOut ro)
 {
     int it = find_item(gstart, nitems, blockIdx.x);
@@ -1357,7 +1466,7 @@ __device__ inline R to_r(double v) { return (R)v; }
 // forward real row transforms: rows y < ny_rows of `in` (row length nxr, zero padded to Lx)
 // -> S[c][y*H + kx]
 template <typename R>
-__global__ void __launch_bounds__(FFT_THREADS) k_rowfwd(const ConvItem* items, const int* gstart,
+__global__ void __launch_bounds__(FFT_THREADS) k_rowfwd(const ConvItem* __restrict__ items, const int* __restrict__ gstart,
                                                         int nitems)
 {
     extern __shared__ char lds_raw[];
@@ -1406,7 +1515,7 @@ __global__ void __launch_bounds__(FFT_THREADS) k_rowfwd(const ConvItem* items, c
 // column stage: forward column FFT of each input, spectral product (mode 0), spectrum store
 // (mode 1) or reciprocal (mode 2), inverse column FFT -> T[c][y*H + kx]
 template <typename R>
-__global__ void __launch_bounds__(FFT_THREADS) k_colmul(const ConvItem* items, const int* gstart,
+__global__ void __launch_bounds__(FFT_THREADS) k_colmul(const ConvItem* __restrict__ items, const int* __restrict__ gstart,
                                                         int nitems)
 {
     extern __shared__ char lds_raw[];
@@ -1480,7 +1589,7 @@ __global__ void __launch_bounds__(FFT_THREADS) k_colmul(const ConvItem* items, c
 
 // inverse real row transforms T[c] -> out[c] rows, masked write (mode 0) or dense (mode 2)
 template <typename R>
-__global__ void __launch_bounds__(FFT_THREADS) k_rowinv(const ConvItem* items, const int* gstart,
+__global__ void __launch_bounds__(FFT_THREADS) k_rowinv(const ConvItem* __restrict__ items, const int* __restrict__ gstart,
                                                         int nitems)
 {
     extern __shared__ char lds_raw[];
@@ -1531,7 +1640,7 @@ __global__ void __launch_bounds__(FFT_THREADS) k_rowinv(const ConvItem* items, c
 // influence coefficients (elascf_pcwcns, src/m_visc.f90:431-604) and their spectra
 // ------------------------------------------------------------------------------------------
 
-__global__ void __launch_bounds__(ELEM_THREADS) k_elascf(const CoefItem* items, const int* gstart, int nitems)
+__global__ void __launch_bounds__(ELEM_THREADS) k_elascf(const CoefItem* __restrict__ items, const int* __restrict__ gstart, int nitems)
 {
     int it = find_item(gstart, nitems, blockIdx.x);
     const CoefItem& I = items[it];
@@ -1620,7 +1729,7 @@ __global__ void k_rollcoef(int n, const double* cs, double* cv)
     }
 }
 
-__global__ void __launch_bounds__(ELEM_THREADS) k_embed(const EmbedItem* items, const int* gstart, int nitems)
+__global__ void __launch_bounds__(ELEM_THREADS) k_embed(const EmbedItem* __restrict__ items, const int* __restrict__ gstart, int nitems)
 {
     int it = find_item(gstart, nitems, blockIdx.x);
     const EmbedItem& I = items[it];
@@ -1638,7 +1747,7 @@ __global__ void __launch_bounds__(ELEM_THREADS) k_embed(const EmbedItem* items, 
     }
 }
 
-__global__ void __launch_bounds__(ELEM_THREADS) k_extract(const ExtractItem* items, const int* gstart, int nitems)
+__global__ void __launch_bounds__(ELEM_THREADS) k_extract(const ExtractItem* __restrict__ items, const int* __restrict__ gstart, int nitems)
 {
     int it = find_item(gstart, nitems, blockIdx.x);
     const ExtractItem& I = items[it];
@@ -1661,7 +1770,7 @@ __global__ void k_to_float(size_t n, const double* in, float* out)
 // per-case fields and force sums
 // ------------------------------------------------------------------------------------------
 
-__global__ void __launch_bounds__(ELEM_THREADS) k_setup(const SetupItem* items, const int* gstart,
+__global__ void __launch_bounds__(ELEM_THREADS) k_setup(const SetupItem* __restrict__ items, const int* __restrict__ gstart,
                                                         int nitems, RedOut ro)
 {
     int it = find_item(gstart, nitems, blockIdx.x);
@@ -1733,7 +1842,7 @@ __global__ void __launch_bounds__(ELEM_THREADS) k_setup(const SetupItem* items, 
     write_partials<2>(acc, 1, ro, gstart, it);
 }
 
-__global__ void __launch_bounds__(ELEM_THREADS) k_forces(const SetupItem* items, const int* gstart,
+__global__ void __launch_bounds__(ELEM_THREADS) k_forces(const SetupItem* __restrict__ items, const int* __restrict__ gstart,
                                                          int nitems, RedOut ro)
 {
     int it = find_item(gstart, nitems, blockIdx.x);
@@ -1760,7 +1869,7 @@ __global__ void __launch_bounds__(ELEM_THREADS) k_forces(const SetupItem* items,
 // (src/m_solvpn.f90:531-650, src/m_solvpt.f90:497-796)
 // ------------------------------------------------------------------------------------------
 
-__global__ void __launch_bounds__(ELEM_THREADS) k_sens(const SensItem* items, const int* gstart,
+__global__ void __launch_bounds__(ELEM_THREADS) k_sens(const SensItem* __restrict__ items, const int* __restrict__ gstart,
                                                        int nitems, RedOut ro)
 {
     int it = find_item(gstart, nitems, blockIdx.x);
@@ -1803,7 +1912,7 @@ __global__ void __launch_bounds__(ELEM_THREADS) k_sens(const SensItem* items, co
 
 // leading edge of transient rolling, sxbnd and stang_rhs (1b) (src/m_leadedge.f90:92-394,
 // src/m_stang.f90:838-935); see LedgeItem
-__global__ void __launch_bounds__(ELEM_THREADS) k_ledge(const LedgeItem* items, const int* gstart,
+__global__ void __launch_bounds__(ELEM_THREADS) k_ledge(const LedgeItem* __restrict__ items, const int* __restrict__ gstart,
                                                         int nitems, RedOut ro)
 {
     int it = find_item(gstart, nitems, blockIdx.x);
@@ -1873,7 +1982,7 @@ constexpr int GS_THREADS = GS_THREADS_N;
 // Rows with an interior element in the trailing-edge column ix = 1: steady rolling then
 // needs ConvexGS (src/m_stang.f90:131-143, 185-190).  One thread per row.  Also returns the
 // tangential coefficients of element (0,0) (blocks xx, xy, yx, yy, unscaled).
-__global__ void __launch_bounds__(ELEM_THREADS) k_guard(const GsItem* items, const int* gstart,
+__global__ void __launch_bounds__(ELEM_THREADS) k_guard(const GsItem* __restrict__ items, const int* __restrict__ gstart,
                                                         int nitems, RedOut ro)
 {
     int it = find_item(gstart, nitems, blockIdx.x);
@@ -1901,7 +2010,7 @@ __global__ void __launch_bounds__(ELEM_THREADS) k_guard(const GsItem* items, con
 // row lives in LDS; dp is written through to global memory for the summation.
 // Returns (itgs, dif, algorithmic flops: 8 per coefficient-difference product of the sums,
 // 0, 0, dif of the first sweep, 0, 0, 0, 0).
-__global__ void __launch_bounds__(GS_THREADS) k_stdygs(const GsItem* items, const int* gstart,
+__global__ void __launch_bounds__(GS_THREADS) k_stdygs(const GsItem* __restrict__ items, const int* __restrict__ gstart,
                                                        int nitems, RedOut ro)
 {
     extern __shared__ double gs_lds[];
@@ -2142,7 +2251,7 @@ __host__ __device__ inline size_t gs2_lds(int mx, int my)
     return gs2_base_lds(mx, my) + (size_t)gs2_stage_rows(mx, my) * gs2_row_lds(mx);
 }
 
-__global__ void __launch_bounds__(GS_THREADS) k_stdygs2(const GsItem* items, const int* gstart,
+__global__ void __launch_bounds__(GS_THREADS) k_stdygs2(const GsItem* __restrict__ items, const int* __restrict__ gstart,
                                                         int nitems, RedOut ro)
 {
     extern __shared__ double gs_lds[];
@@ -2579,13 +2688,6 @@ struct GsRow {
 // (quad permutes [1,0,3,2] and [2,3,0,1], then the half-row and row mirrors: every lane of a
 // row ends with the row's sum, the same bits by commutativity), then the four row sums read
 // from lanes 0, 16, 32, 48 and added in that order.  Needs all 64 lanes active.
-template <int CTRL>
-__device__ inline double dpp_f64(double v)
-{
-    const int lo = __builtin_amdgcn_update_dpp(0, __double2loint(v), CTRL, 0xF, 0xF, false);
-    const int hi = __builtin_amdgcn_update_dpp(0, __double2hiint(v), CTRL, 0xF, 0xF, false);
-    return __hiloint2double(hi, lo);
-}
 __device__ inline double lane_f64(double v, int l)
 {
     return __hiloint2double(__builtin_amdgcn_readlane(__double2hiint(v), l),
@@ -2800,7 +2902,7 @@ __host__ __device__ inline size_t gs3_lds(int mx, int my)
     return gs3_stage_off(mx, my) + 2 * (size_t)gs3_stage_stride(mx) * sizeof(double);
 }
 
-__global__ void __launch_bounds__(GS_THREADS) k_stdygs3(const GsItem* items, const int* gstart,
+__global__ void __launch_bounds__(GS_THREADS) k_stdygs3(const GsItem* __restrict__ items, const int* __restrict__ gstart,
                                                         int nitems, RedOut ro)
 {
     extern __shared__ double gs_lds[];
@@ -3136,7 +3238,7 @@ constexpr int GSB_THREADS = 256;
 // set-up: dp = differences along x (the leading-edge column keeps p, src/m_solvpt.f90:
 // 2893-2908), the summation and interior range of each row, d = 0 and the sweep state.
 // Returns (first interior row, last interior row, summed range lengths).
-__global__ void __launch_bounds__(GSB_THREADS) k_gsb_setup(const GsbItem* items, const int* gstart,
+__global__ void __launch_bounds__(GSB_THREADS) k_gsb_setup(const GsbItem* __restrict__ items, const int* __restrict__ gstart,
                                                            int nitems, RedOut ro)
 {
     __shared__ double red[16 * MAXK];
@@ -3209,7 +3311,7 @@ __host__ __device__ inline size_t gsb_lds(int mx)
 // walks the row with the own-row influence of the current differences, as k_stdygs3 does.
 // The row products run on all threads: a thread owns GS3_TB consecutive targets and takes
 // the sources in chunks of GS3_QB from one coefficient window per block (xx, xy = yx, yy).
-__global__ void __launch_bounds__(GSB_THREADS) k_gsb_walk(const GsbItem* items, const int* gstart,
+__global__ void __launch_bounds__(GSB_THREADS) k_gsb_walk(const GsbItem* __restrict__ items, const int* __restrict__ gstart,
                                                           int nitems, RedOut ro)
 {
     extern __shared__ double gsb_lds_[];
@@ -3419,7 +3521,7 @@ __global__ void __launch_bounds__(GSB_THREADS) k_gsb_walk(const GsbItem* items, 
 // end of a sweep (src/m_solvpt.f90:3130-3150): dif = sqrt(sum |dp|^2 / 2k), difid from the rms
 // of p (of p - p0 in a sensitivity solve); counts the sweep and clears its sum.  Returns
 // (itgs, dif, flops, 0, 0, dif1, still sweeping, difid, 0, 0).
-__global__ void __launch_bounds__(GSB_THREADS) k_gsb_check(const GsbItem* items, const int* gstart,
+__global__ void __launch_bounds__(GSB_THREADS) k_gsb_check(const GsbItem* __restrict__ items, const int* __restrict__ gstart,
                                                            int nitems, RedOut ro)
 {
     __shared__ double red[16 * MAXK];
@@ -3464,7 +3566,7 @@ __global__ void __launch_bounds__(GSB_THREADS) k_gsb_check(const GsbItem* items,
 
 // One wavefront per patch runs every sweep (the element updates are sequential; each shift is
 // a direct sum over the interior elements, split over the 64 lanes and reduced by shuffles).
-__global__ void __launch_bounds__(64) k_cnvxgs(const CgsItem* items, const int* gstart, int nitems,
+__global__ void __launch_bounds__(64) k_cnvxgs(const CgsItem* __restrict__ items, const int* __restrict__ gstart, int nitems,
                                                RedOut ro)
 {
     int it = find_item(gstart, nitems, blockIdx.x);
@@ -3609,7 +3711,7 @@ typedef double dense_v4 __attribute__((ext_vector_type(4)));
 // the d range (a serial chain an eighth as long); wavefront 0 adds the parts in wave order.
 constexpr int DENSE_WAVES = 8;
 
-__global__ void __launch_bounds__(64 * DENSE_WAVES) k_dense(const DenseItem* items, const int* gstart, int nitems)
+__global__ void __launch_bounds__(64 * DENSE_WAVES) k_dense(const DenseItem* __restrict__ items, const int* __restrict__ gstart, int nitems)
 {
     __shared__ double part[DENSE_WAVES][3][4][64];
     const int it = find_item(gstart, nitems, blockIdx.x);
