@@ -6,6 +6,7 @@
 #include <hip/hip_runtime.h>
 
 #include <cmath>
+#include <cstdint>
 #include <cstdio>
 
 #include "fft_core.hpp"
@@ -33,6 +34,15 @@ __device__ inline int find_item(const int* gstart, int nitems, int g)
         else hi = mid - 1;
     }
     return lo;
+}
+
+// A pointer read from an item record is generic to the compiler, which then makes flat loads and
+// stores of it: these count on the LDS counter too, so that every LDS access near them waits for
+// memory.  The grid functions are all in global memory.
+template <typename T>
+__device__ inline __attribute__((address_space(1))) T* as_global(T* p)
+{
+    return (__attribute__((address_space(1))) T*)(uintptr_t)p;
 }
 
 __device__ inline bool in_mask(int mask, int8_t e)
@@ -799,8 +809,9 @@ __global__ void __launch_bounds__(ELEM_THREADS) k_st_sa(const StItem* __restrict
 // it loads the recurrence inputs with coalesced reads into LDS, one thread per row runs the
 // recurrence in LDS, and the element-wise rest is done by all threads with coalesced access.
 constexpr int GD_THREADS = 256;
-constexpr int GD_TILE = 2048;          // elements per tile (probe, update)
-constexpr int GD_TILE_PROJ = 1024;     // elements per tile (project)
+constexpr int GD_ROW_THREADS = 256;    // threads of update and project
+constexpr int GD_TILE = 2048;          // elements per tile (probe; its sums follow this shape)
+constexpr int GD_TILE_ROW = 1024;      // elements per tile (update, project)
 
 __host__ __device__ inline int gd_rows_per_tile(int mx, int my, int tile)
 {
@@ -810,6 +821,119 @@ __host__ __device__ inline int gd_rows_per_tile(int mx, int my, int tile)
     return r < my ? r : my;
 }
 __host__ __device__ inline int gd_row_stride(int mx) { return mx | 1; }
+
+// Cells of the LDS tiles of the row recurrences: two components side by side; and for
+// apply_trcbnd the bound with the state in its sign (adhesion g, slip -g, exterior +inf; GD has
+// no other states) and the least |p|^2 at which the bound has to be looked at (in adhesion
+// below g^2 by more than the rounding of a square root: p2 < lim implies sqrt(p2) < g).
+struct GdCell {
+    double x, y;
+};
+struct GdBound {
+    double c, lim;
+};
+__device__ inline GdBound gd_bound(double g, int8_t st)
+{
+    if (st == ADHES) return GdBound{g, g * g * (1.0 - 0x1p-50)};
+    return st == SLIP ? GdBound{-g, -1.0} : GdBound{INFINITY, INFINITY};
+}
+__device__ inline int8_t gd_state(const GdBound& b)
+{
+    return b.c == INFINITY ? EXTER : (b.lim < 0.0 ? SLIP : ADHES);
+}
+
+// apply_trcbnd along one row (src/gdsteady.f90:807-847): from the leading edge, p = p(ix+1) + dp,
+// put on the bound in slip and where it exceeds it.  lp holds dp and receives p.  One lane per
+// row, so the row's chain of dependent operations is the kernel's time (FP64 operations issue
+// 10 cycles after the one they need, sqrt takes 112, a division 75, an LDS read 60, a divergent
+// branch 30).  The cells are read from LDS four ahead of their use; a step in which every row
+// of the wave is in the exterior or below its bound ends after one comparison; there is no
+// other branch in the usual range.
+//   p g / |p|: the square root is the correctly rounded one (two corrections of the hardware
+// estimate); the half reciprocal left over from it needs one correction to start the two
+// divisions, and each ends with the residual correction that rounds it correctly: the bits of
+// px * g / sqrt(px * px + py * py) without the range handling of the general sequences, which
+// serve the steps where |p|^2 leaves 2^+-600.  A step in slip takes about 300 cycles so, with the
+// compiler's square root and divisions and the reads in place 580 (k_gd_probe of one 512 x 512
+// patch: 121 us a launch, then 90; 1024 x 1024: 175 and 139 us; 40 x 40: 22.6 and 20.3 us).
+__device__ inline void trcbnd_row(GdCell* lp, const GdBound* lb, int mx)
+{
+    constexpr int U = 4;
+    lp[mx - 1] = GdCell{0.0, 0.0};
+    double pxn = 0.0, pyn = 0.0;
+    auto step = [&](const GdCell d, const GdBound b, int ix) {
+        double px = pxn + d.x, py = pyn + d.y;
+        const double p2 = fma(px, px, py * py);
+        const bool need = !(p2 < b.lim);
+        if (__builtin_amdgcn_ballot_w64(need)) {
+            const double g = fabs(b.c), nx = px * g, ny = py * g;
+            const bool wide = (unsigned)(__double2hiint(p2) - (423 << 20)) >= (1200u << 20);
+            if (__builtin_amdgcn_ballot_w64(need && wide)) {
+                const double s = sqrt(p2);
+                if (need && s >= b.c) {
+                    px = nx / s;
+                    py = ny / s;
+                }
+            } else {
+                const double y = __builtin_amdgcn_rsq(p2);
+                double s = p2 * y, h = 0.5 * y;
+                const double r = fma(-h, s, 0.5);
+                s = fma(s, r, s);
+                h = fma(h, r, h);
+                s = fma(fma(-s, s, p2), h, s);
+                s = fma(fma(-s, s, p2), h, s);
+                double q = h + h;
+                q = fma(q, fma(-s, q, 1.0), q);
+                const double qx = nx * q, qy = ny * q;
+                const bool clip = s >= b.c;   // (true in slip, false in the exterior)
+                const double ex = copysign(fma(fma(-s, qx, nx), q, qx), nx);
+                const double ey = copysign(fma(fma(-s, qy, ny), q, qy), ny);
+                px = clip ? ex : px;
+                py = clip ? ey : py;
+            }
+        }
+        const bool ext = __double2hiint(b.c) == 0x7FF00000;
+        pxn = ext ? 0.0 : px;
+        pyn = ext ? 0.0 : py;
+        lp[ix] = GdCell{pxn, pyn};
+    };
+    int ix = mx - 2;
+    // the first (mx - 1) mod 2 U elements singly, then two sets of U registers in turn
+    for (; (ix + 1) % (2 * U) != 0; ix--) step(lp[ix], lb[ix], ix);
+    if (ix < 0) return;
+    GdCell d[U], e[U];
+    GdBound c[U], f[U];
+#pragma unroll
+    for (int u = 0; u < U; u++) {
+        d[u] = lp[ix - u];
+        c[u] = lb[ix - u];
+    }
+    for (; ix >= 0; ix -= 2 * U) {
+        const int i1 = ix - U, i2 = ix >= 2 * U ? ix - 2 * U : i1;   // (the last set is not used)
+#pragma unroll
+        for (int u = 0; u < U; u++) {
+            e[u] = lp[i1 - u];
+            f[u] = lb[i1 - u];
+        }
+#pragma unroll
+        for (int u = 0; u < U; u++) step(d[u], c[u], ix - u);
+#pragma unroll
+        for (int u = 0; u < U; u++) {
+            d[u] = lp[i2 - u];
+            c[u] = lb[i2 - u];
+        }
+#pragma unroll
+        for (int u = 0; u < U; u++) step(e[u], f[u], i1 - u);
+    }
+}
+
+// The row of a tile that this thread recurs along, from 0; beyond the tile's rows: none.  The
+// lanes of one wave (or its neighbours, for more than 64 rows) do; which wave that is changes
+// with the group, so that the chains of the groups that share a CU run on different SIMDs.
+__device__ inline int gd_chain_row()
+{
+    return (threadIdx.x + blockDim.x - ((blockIdx.x >> 8) & 3) * 64) % blockDim.x;
+}
 
 // compute_dp, src/gdsteady.f90:610-635: dp = backward differences along x (element-wise)
 __global__ void __launch_bounds__(ELEM_THREADS) k_gd_dp(const GdItem* __restrict__ items, const int* __restrict__ gstart,
@@ -832,110 +956,157 @@ __global__ void __launch_bounds__(ELEM_THREADS) k_gd_dp(const GdItem* __restrict
     }
 }
 
-// project_searchdir, src/gdsteady.f90:639-803: dv from the residual r, with v // t in slip
-__global__ void __launch_bounds__(GD_THREADS) k_gd_project(const GdItem* __restrict__ items, const int* __restrict__ gstart,
-                                                           int nitems, RedOut ro)
+// project_searchdir, src/gdsteady.f90:639-803: dv from the residual r, with v // t in slip.
+// In slip and in the exterior v does not depend on the row's other elements, so all threads
+// form it while loading; what is left for the one lane per row is v = v(ix+1) + r in adhesion,
+// with the elements read four ahead; dv = v - v(ix+1) follows element-wise.  One patch of
+// 1024 x 1024: 470 us a launch with everything in the row loop (a dependent LDS round trip for
+// each of three reads an element), 102 us so; 512 x 512: 129 and 37 us; 40 x 40: 18 and 10 us.
+// (512 threads a group: 36 and 9.8 us on the smaller two, but 131 us on the largest, where half
+// as many rows are then on the chip.)
+__global__ void __launch_bounds__(GD_ROW_THREADS, 4) k_gd_project(const GdItem* __restrict__ items, const int* __restrict__ gstart,
+                                                               int nitems, RedOut ro)
 {
     extern __shared__ double gd_lds[];
     int it = find_item(gstart, nitems, blockIdx.x);
     const GdItem& I = items[it];
     const int mx = I.mx, S = gd_row_stride(mx);
-    const int R = gd_rows_per_tile(mx, I.my, GD_TILE_PROJ);
+    const int R = gd_rows_per_tile(mx, I.my, GD_TILE_ROW);
     const int row0 = (blockIdx.x - gstart[it]) * R;
     const int nrow = min(R, I.my - row0);
     const int ne = nrow * mx;
     const size_t g0 = (size_t)row0 * mx;
-    double* lrx = gd_lds;
-    double* lry = lrx + R * S;
-    double* lg = lry + R * S;
-    double* lnx = lg + R * S;        // n, then v
-    double* lny = lnx + R * S;
-    double* ldx = lny + R * S;       // dv
-    double* ldy = ldx + R * S;
-    int8_t* lel = (int8_t*)(ldy + R * S);
-    for (int e = threadIdx.x; e < ne; e += GD_THREADS) {
-        int r = e / mx, l = r * S + (e - r * mx);
-        size_t i = g0 + e;
-        int8_t st = I.el[i];
-        lel[l] = st;
-        lrx[l] = I.rx[i];
-        lry[l] = I.ry[i];
-        if (st == SLIP) {
-            lg[l] = I.mu * I.pn[i];
-            lnx[l] = I.nx[i];
-            lny[l] = I.ny[i];
+    GdCell* lv = (GdCell*)gd_lds;    // r in adhesion, v elsewhere; then v
+    GdCell* lr = lv + R * S;         // r (E_down only)
+    int8_t* lel = (int8_t*)(lr + R * S);
+    const int imeth = I.imeth, kdown = I.kdown;
+    const double fdecay = I.fdecay;
+    // a tile has at most U x GD_ROW_THREADS elements (grids have at most 2048 columns)
+    constexpr int U = 2048 / GD_ROW_THREADS;
+    int8_t st[U];
+    double rx[U], ry[U], nx[U], ny[U], pn[U], vt[U];
+#pragma unroll
+    for (int u = 0; u < U; u++) {
+        if (u * GD_ROW_THREADS >= ne) break;
+        const int e = threadIdx.x + u * GD_ROW_THREADS;
+        const size_t i = g0 + (e < ne ? e : 0);
+        st[u] = as_global(I.el)[i];
+        rx[u] = as_global(I.rx)[i];
+        ry[u] = as_global(I.ry)[i];
+        nx[u] = as_global(I.nx)[i];
+        ny[u] = as_global(I.ny)[i];
+        pn[u] = as_global(I.pn)[i];
+    }
+#pragma unroll
+    for (int u = 0; u < U; u++) {
+        if (u * GD_ROW_THREADS >= ne) break;
+        const int e = threadIdx.x + u * GD_ROW_THREADS;
+        const int r = e / mx, ix = e - r * mx, l = r * S + ix;
+        const double g = I.mu * pn[u];
+        const double tx = -ny[u], ty = nx[u];
+        const double w = tx * rx[u] + ty * ry[u];
+        vt[u] = copysign(1.0, w) * fmin(fabs(w), I.fac_v * g);
+        GdCell v{0.0, 0.0};
+        if (ix != mx - 1) {
+            if (st[u] == SLIP) v = GdCell{tx * vt[u], ty * vt[u]};
+            else if (st[u] == ADHES) v = GdCell{rx[u], ry[u]};
+        }
+        if (e < ne) {
+            lel[l] = st[u];
+            lv[l] = v;
+            if (imeth == 2) lr[l] = GdCell{rx[u], ry[u]};
         }
     }
     __syncthreads();
-    if (threadIdx.x < nrow) {
-        const int l0 = threadIdx.x * S;
-        const int imeth = I.imeth, kdown = I.kdown;
+    if (const int row = gd_chain_row(); row < nrow) {
+        GdCell* const v = lv + row * S;
+        const int8_t* const el = lel + row * S;
         double vxn = 0.0, vyn = 0.0;   // v at ix+1
-        lnx[l0 + mx - 1] = 0.0;
-        lny[l0 + mx - 1] = 0.0;
-        ldx[l0 + mx - 1] = lrx[l0 + mx - 1];
-        ldy[l0 + mx - 1] = lry[l0 + mx - 1];
-        int last_se = 1 << 30;   // smallest processed (1-based) ix in slip/exterior, E_down
-        for (int ix = mx - 2; ix >= 0; ix--) {
-            const int l = l0 + ix;
-            int8_t st = lel[l];
-            double dvx = lrx[l], dvy = lry[l], vx, vy;
-            if (st == ADHES) {
-                if (imeth == 1) {
-                    vx = vxn + dvx;
-                    vy = vyn + dvy;
-                } else if (imeth == 3) {
-                    vx = I.fdecay * vxn + dvx;
-                    vy = I.fdecay * vyn + dvy;
-                    dvx = vx - vxn;
-                    dvy = vy - vyn;
-                } else {
-                    int ixf = ix + 1;
+        if (imeth == 2) {
+            const GdCell* const r = lr + row * S;
+            int last_se = 1 << 30;   // smallest processed (1-based) ix in slip/exterior, E_down
+            for (int ix = mx - 2; ix >= 0; ix--) {
+                GdCell c = v[ix];
+                if (el[ix] == ADHES) {
+                    const int ixf = ix + 1;
+                    c.x = vxn + c.x;
+                    c.y = vyn + c.y;
                     if (ixf + kdown <= mx) {
-                        double inx = lrx[l + kdown], iny = lry[l + kdown];
-                        if (last_se <= ixf + kdown - 1) { inx = 0.0; iny = 0.0; }
-                        vx = vxn + dvx - inx;
-                        vy = vyn + dvy - iny;
-                    } else {
-                        vx = vxn + dvx;
-                        vy = vyn + dvy;
+                        GdCell in = r[ix + kdown];
+                        if (last_se <= ixf + kdown - 1) in = GdCell{0.0, 0.0};
+                        c.x = c.x - in.x;
+                        c.y = c.y - in.y;
                     }
-                    dvx = vx - vxn;
-                    dvy = vy - vyn;
+                    v[ix] = c;
+                } else {
+                    last_se = ix + 1;
                 }
-            } else if (st == SLIP) {
-                double g = lg[l];
-                double tx = -lny[l], ty = lnx[l];
-                double vt = tx * dvx + ty * dvy;
-                vt = copysign(1.0, vt) * fmin(fabs(vt), I.fac_v * g);
-                vx = tx * vt;
-                vy = ty * vt;
-                dvx = vx - vxn;
-                dvy = vy - vyn;
-                last_se = ix + 1;
-            } else {
-                vx = 0.0;
-                vy = 0.0;
-                dvx = -vxn;
-                dvy = -vyn;
-                last_se = ix + 1;
+                vxn = c.x;
+                vyn = c.y;
             }
-            lnx[l] = vx;
-            lny[l] = vy;
-            ldx[l] = dvx;
-            ldy[l] = dvy;
-            vxn = vx;
-            vyn = vy;
+        } else {
+            // v = f v(ix+1) + r in adhesion, f = 1 (the bits of the sum) or fdecay
+            constexpr int V = 4;
+            const double f = imeth == 3 ? fdecay : 1.0;
+            auto step = [&](const GdCell c, int8_t e, int ix) {
+                const double ax = fma(f, vxn, c.x), ay = fma(f, vyn, c.y);
+                vxn = e == ADHES ? ax : c.x;
+                vyn = e == ADHES ? ay : c.y;
+                if (e == ADHES) v[ix] = GdCell{vxn, vyn};
+            };
+            int ix = mx - 2;
+            for (; (ix + 1) % (2 * V) != 0; ix--) step(v[ix], el[ix], ix);
+            GdCell c[V], d[V];
+            int8_t e[V], k[V];
+            if (ix >= 0)
+#pragma unroll
+                for (int u = 0; u < V; u++) {
+                    c[u] = v[ix - u];
+                    e[u] = el[ix - u];
+                }
+            for (; ix >= 0; ix -= 2 * V) {
+                const int i1 = ix - V, i2 = ix >= 2 * V ? ix - 2 * V : i1;   // (the last set is not used)
+#pragma unroll
+                for (int u = 0; u < V; u++) {
+                    d[u] = v[i1 - u];
+                    k[u] = el[i1 - u];
+                }
+#pragma unroll
+                for (int u = 0; u < V; u++) step(c[u], e[u], ix - u);
+#pragma unroll
+                for (int u = 0; u < V; u++) {
+                    c[u] = v[i2 - u];
+                    e[u] = el[i2 - u];
+                }
+#pragma unroll
+                for (int u = 0; u < V; u++) step(d[u], k[u], i1 - u);
+            }
         }
     }
     __syncthreads();
-    for (int e = threadIdx.x; e < ne; e += GD_THREADS) {
-        int r = e / mx, l = r * S + (e - r * mx);
-        size_t i = g0 + e;
-        I.vx[i] = lnx[l];
-        I.vy[i] = lny[l];
-        I.dvx[i] = ldx[l];
-        I.dvy[i] = ldy[l];
+#pragma unroll
+    for (int u = 0; u < U; u++) {
+        const int e = threadIdx.x + u * GD_ROW_THREADS;
+        if (e >= ne) break;
+        const int r = e / mx, ix = e - r * mx, l = r * S + ix;
+        const size_t i = g0 + e;
+        const GdCell v = lv[l];
+        double dvx = rx[u], dvy = ry[u];
+        // the leading-edge column and adhesion with the plain recurrence keep dv = r
+        if (ix != mx - 1 && !(st[u] == ADHES && imeth == 1)) {
+            const GdCell n = lv[l + 1];
+            if (st[u] == SLIP) {
+                dvx = fma(vt[u], -ny[u], -n.x);
+                dvy = fma(nx[u], vt[u], -n.y);
+            } else {
+                dvx = v.x - n.x;
+                dvy = v.y - n.y;
+            }
+        }
+        as_global(I.vx)[i] = v.x;
+        as_global(I.vy)[i] = v.y;
+        as_global(I.dvx)[i] = dvx;
+        as_global(I.dvy)[i] = dvy;
     }
 }
 
@@ -956,59 +1127,76 @@ __global__ void __launch_bounds__(GD_THREADS) k_gd_probe(const GdItem* __restric
     const int ne = nrow * mx;
     const size_t g0 = (size_t)row0 * mx;
     const double a = I.alpha;
-    double* lpx = gd_lds;            // dp + alpha dv, then the new p
-    double* lpy = lpx + R * S;
-    double* lg = lpy + R * S;
-    int8_t* lel = (int8_t*)(lg + R * S);
-    for (int e = threadIdx.x; e < ne; e += GD_THREADS) {
-        int r = e / mx, l = r * S + (e - r * mx);
-        size_t i = g0 + e;
-        int8_t st = I.el[i];
-        lel[l] = st;
-        if (st >= ADHES) {
-            lg[l] = I.mu * I.pn[i];
-            lpx[l] = I.dpx[i] + a * I.dvx[i];
-            lpy[l] = I.dpy[i] + a * I.dvy[i];
+    GdCell* lp = (GdCell*)gd_lds;    // dp + alpha dv, then the new p
+    GdBound* lb = (GdBound*)(lp + R * S);
+    constexpr int U = 4;
+    for (int e0 = threadIdx.x; e0 < ne; e0 += U * GD_THREADS) {
+        int8_t st[U];
+        double pn[U], dx[U], dy[U], vx[U], vy[U];
+#pragma unroll
+        for (int u = 0; u < U; u++) {
+            const int e = e0 + u * GD_THREADS;
+            const size_t i = g0 + (e < ne ? e : 0);
+            st[u] = as_global(I.el)[i];
+            pn[u] = as_global(I.pn)[i];
+            dx[u] = as_global(I.dpx)[i];
+            dy[u] = as_global(I.dpy)[i];
+            vx[u] = as_global(I.dvx)[i];
+            vy[u] = as_global(I.dvy)[i];
+        }
+#pragma unroll
+        for (int u = 0; u < U; u++) {
+            const int e = e0 + u * GD_THREADS;
+            const int r = e / mx, l = r * S + (e - r * mx);
+            const GdCell c{fma(a, vx[u], dx[u]), fma(a, vy[u], dy[u])};
+            const GdBound b = gd_bound(I.mu * pn[u], st[u]);
+            if (e < ne) {
+                lp[l] = c;
+                lb[l] = b;
+            }
         }
     }
+    // the element terms' inputs: the first element's are on their way during the row recurrence,
+    // then each element's during the arithmetic of the one before
+    struct Terms {
+        double dscl, sx, sy, qx, qy, rx, ry, nx, ny, vx, vy;
+    };
+    const int first = I.first;
+    auto fetch = [&](int e) {
+        const size_t ii = g0 + (e < ne ? e : 0);
+        Terms t;
+        t.dscl = as_global(I.dscl)[ii];
+        t.sx = as_global(I.sx)[ii];
+        t.sy = as_global(I.sy)[ii];
+        t.qx = as_global(I.qx)[ii];
+        t.qy = as_global(I.qy)[ii];
+        t.rx = first ? as_global(I.rx)[ii] : 0.0;
+        t.ry = first ? as_global(I.ry)[ii] : 0.0;
+        t.nx = as_global(I.nx)[ii];
+        t.ny = as_global(I.ny)[ii];
+        t.vx = as_global(I.vx)[ii];
+        t.vy = as_global(I.vy)[ii];
+        return t;
+    };
+    Terms ahead = fetch(threadIdx.x);
     __syncthreads();
-    if (threadIdx.x < nrow) {
-        const int l0 = threadIdx.x * S;
-        double pxn = 0.0, pyn = 0.0;   // new p at ix+1
-        for (int ix = mx - 1; ix >= 0; ix--) {
-            const int l = l0 + ix;
-            int8_t st = lel[l];
-            double px, py;
-            if (ix == mx - 1 || st <= EXTER) {
-                px = 0.0;
-                py = 0.0;
-            } else {
-                double g = lg[l];
-                px = pxn + lpx[l];
-                py = pyn + lpy[l];
-                double ptabs = sqrt(px * px + py * py);
-                if (st == SLIP || ptabs >= g) {
-                    px = px * g / ptabs;
-                    py = py * g / ptabs;
-                }
-            }
-            lpx[l] = px;
-            lpy[l] = py;
-            pxn = px;
-            pyn = py;
-        }
+    if (const int row = gd_chain_row(); row < nrow) {
+        const int l0 = row * S;
+        trcbnd_row(lp + l0, lb + l0, mx);
     }
     __syncthreads();
     double acc[10] = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
     const double tiny = 1e-12;
     for (int e = threadIdx.x; e < ne; e += GD_THREADS) {
         int r = e / mx, l = r * S + (e - r * mx);
-        size_t ii = g0 + e;
-        int8_t st = lel[l];
-        double dscl = I.dscl[ii];
-        double sx = I.sx[ii], sy = I.sy[ii], qx = I.qx[ii], qy = I.qy[ii];
-        if (I.first) {
-            double rx = I.rx[ii], ry = I.ry[ii];
+        const GdBound b = lb[l];
+        const int8_t st = gd_state(b);
+        const Terms t = ahead;
+        if (e + GD_THREADS < ne) ahead = fetch(e + GD_THREADS);
+        double dscl = t.dscl;
+        double sx = t.sx, sy = t.sy, qx = t.qx, qy = t.qy;
+        if (first) {
+            double rx = t.rx, ry = t.ry;
             acc[6] += rx * rx + ry * ry;
             acc[7] += (rx * qx + ry * qy) * dscl;
             if (st >= ADHES) {
@@ -1017,9 +1205,9 @@ __global__ void __launch_bounds__(GD_THREADS) k_gd_probe(const GdItem* __restric
             }
         }
         if (st != ADHES && st != SLIP) continue;
-        double px = lpx[l], py = lpy[l], g = lg[l];
-        double txo = -I.ny[ii], tyo = I.nx[ii];
-        double vt = I.vx[ii] * txo + I.vy[ii] * tyo;
+        double px = lp[l].x, py = lp[l].y, g = fabs(b.c);
+        double txo = -t.ny, tyo = t.nx;
+        double vt = t.vx * txo + t.vy * tyo;
         double dth_da = (g * vt) / (fmax(tiny, g * g) + a * a * vt * vt);
         double nxn, nyn;
         nt_from_p(px, py, nxn, nyn);
@@ -1046,86 +1234,80 @@ __global__ void __launch_bounds__(GD_THREADS) k_gd_probe(const GdItem* __restric
     write_partials<10>(acc, 0, ro, gstart, it);
 }
 
-// pold = p; dp += alpha dv on the interior; apply_trcbnd (src/gdsteady.f90:807-847); n from p
-__global__ void __launch_bounds__(GD_THREADS) k_gd_update(const GdItem* __restrict__ items, const int* __restrict__ gstart,
-                                                          int nitems, RedOut ro)
+// pold = p; dp += alpha dv on the interior; apply_trcbnd (src/gdsteady.f90:807-847); n from p.
+// No sums, so tiles and threads are free of the probe's: half its tile, so that every CU has one
+// at 512 x 512: 118 us a launch with the plain row loop in the probe's tile, 73 us so; 1024 x
+// 1024: 171 and 162 us; 40 x 40: 22 and 16 us.
+__global__ void __launch_bounds__(GD_ROW_THREADS, 4) k_gd_update(const GdItem* __restrict__ items, const int* __restrict__ gstart,
+                                                              int nitems, RedOut ro)
 {
     extern __shared__ double gd_lds[];
     int it = find_item(gstart, nitems, blockIdx.x);
     const GdItem& I = items[it];
     const int mx = I.mx, S = gd_row_stride(mx);
-    const int R = gd_rows_per_tile(mx, I.my, GD_TILE);
+    const int R = gd_rows_per_tile(mx, I.my, GD_TILE_ROW);
     const int row0 = (blockIdx.x - gstart[it]) * R;
     const int nrow = min(R, I.my - row0);
     const int ne = nrow * mx;
     const size_t g0 = (size_t)row0 * mx;
-    double* lpx = gd_lds;            // dp + alpha dv, then the new p
-    double* lpy = lpx + R * S;
-    double* lg = lpy + R * S;
-    int8_t* lel = (int8_t*)(lg + R * S);
-    for (int e = threadIdx.x; e < ne; e += GD_THREADS) {
-        int r = e / mx, l = r * S + (e - r * mx);
-        size_t i = g0 + e;
-        int8_t st = I.el[i];
-        lel[l] = st;
-        lg[l] = I.mu * I.pn[i];
-        double dpx = I.dpx[i], dpy = I.dpy[i];
-        if (st >= ADHES) {
-            dpx += I.alpha * I.dvx[i];
-            dpy += I.alpha * I.dvy[i];
+    GdCell* lp = (GdCell*)gd_lds;    // dp + alpha dv, then the new p
+    GdBound* lb = (GdBound*)(lp + R * S);
+    constexpr int U = 2;
+    for (int e0 = threadIdx.x; e0 < ne; e0 += U * GD_ROW_THREADS) {
+        int8_t st[U];
+        double pn[U], dx[U], dy[U], vx[U], vy[U], px[U], py[U];
+#pragma unroll
+        for (int u = 0; u < U; u++) {
+            const int e = e0 + u * GD_ROW_THREADS;
+            const size_t i = g0 + (e < ne ? e : 0);
+            st[u] = as_global(I.el)[i];
+            pn[u] = as_global(I.pn)[i];
+            dx[u] = as_global(I.dpx)[i];
+            dy[u] = as_global(I.dpy)[i];
+            vx[u] = as_global(I.dvx)[i];
+            vy[u] = as_global(I.dvy)[i];
+            px[u] = as_global(I.px)[i];
+            py[u] = as_global(I.py)[i];
         }
-        lpx[l] = dpx;
-        lpy[l] = dpy;
-        I.poldx[i] = I.px[i];
-        I.poldy[i] = I.py[i];
-        // the leading-edge column keeps dp (not recomputed from p)
-        if (e - r * mx == mx - 1) {
-            I.dpx[i] = dpx;
-            I.dpy[i] = dpy;
-        }
-    }
-    __syncthreads();
-    if (threadIdx.x < nrow) {
-        const int l0 = threadIdx.x * S;
-        double pxn = 0.0, pyn = 0.0;
-        for (int ix = mx - 1; ix >= 0; ix--) {
-            const int l = l0 + ix;
-            int8_t st = lel[l];
-            double px, py;
-            if (ix == mx - 1 || st <= EXTER) {
-                px = 0.0;
-                py = 0.0;
-            } else {
-                double g = lg[l];
-                px = pxn + lpx[l];
-                py = pyn + lpy[l];
-                double ptabs = sqrt(px * px + py * py);
-                if (st == SLIP || ptabs >= g) {
-                    px = px * g / ptabs;
-                    py = py * g / ptabs;
-                }
+#pragma unroll
+        for (int u = 0; u < U; u++) {
+            const int e = e0 + u * GD_ROW_THREADS;
+            if (e >= ne) break;
+            const int r = e / mx, ix = e - r * mx, l = r * S + ix;
+            const size_t i = g0 + e;
+            GdCell c{dx[u], dy[u]};
+            if (st[u] >= ADHES) c = GdCell{fma(I.alpha, vx[u], dx[u]), fma(I.alpha, vy[u], dy[u])};
+            lp[l] = c;
+            lb[l] = gd_bound(I.mu * pn[u], st[u]);
+            as_global(I.poldx)[i] = px[u];
+            as_global(I.poldy)[i] = py[u];
+            // the leading-edge column keeps dp (not recomputed from p)
+            if (ix == mx - 1) {
+                as_global(I.dpx)[i] = c.x;
+                as_global(I.dpy)[i] = c.y;
             }
-            lpx[l] = px;
-            lpy[l] = py;
-            pxn = px;
-            pyn = py;
         }
     }
     __syncthreads();
-    for (int e = threadIdx.x; e < ne; e += GD_THREADS) {
-        int r = e / mx, ix = e - r * mx, l = r * S + ix;
-        size_t ii = g0 + e;
-        double px = lpx[l], py = lpy[l];
+    if (const int row = gd_chain_row(); row < nrow) {
+        const int l0 = row * S;
+        trcbnd_row(lp + l0, lb + l0, mx);
+    }
+    __syncthreads();
+    for (int e = threadIdx.x; e < ne; e += GD_ROW_THREADS) {
+        const int r = e / mx, ix = e - r * mx, l = r * S + ix;
+        const size_t ii = g0 + e;
+        const GdCell p = lp[l];
         if (ix != mx - 1) {
-            I.dpx[ii] = px - lpx[l + 1];
-            I.dpy[ii] = py - lpy[l + 1];
+            as_global(I.dpx)[ii] = p.x - lp[l + 1].x;
+            as_global(I.dpy)[ii] = p.y - lp[l + 1].y;
         }
-        I.px[ii] = px;
-        I.py[ii] = py;
+        as_global(I.px)[ii] = p.x;
+        as_global(I.py)[ii] = p.y;
         double nx, ny;
-        nt_from_p(px, py, nx, ny);
-        I.nx[ii] = nx;
-        I.ny[ii] = ny;
+        nt_from_p(p.x, p.y, nx, ny);
+        as_global(I.nx)[ii] = nx;
+        as_global(I.ny)[ii] = ny;
     }
 }
 
@@ -3827,6 +4009,7 @@ __global__ void __launch_bounds__(64 * DENSE_WAVES) k_dense(const DenseItem* __r
 // ------------------------------------------------------------------------------------------
 
 static int ngroups_elem(int n) { return (n + ELEM_THREADS * ELEM_PER_THREAD - 1) / (ELEM_THREADS * ELEM_PER_THREAD); }
+static int gd_tile(int kind) { return kind == OP_GD_PROBE ? GD_TILE : GD_TILE_ROW; }
 static int ngroups_rows(int my) { return (my + ROW_THREADS - 1) / ROW_THREADS; }
 
 int op_nred(int kind, const void* item)
@@ -3889,7 +4072,7 @@ int op_groups(int kind, const void* item, int conv_stage)
     case OP_GD_DP: return ngroups_elem(((const GdItem*)item)->n);
     case OP_GD_PROJECT: case OP_GD_PROBE: case OP_GD_UPDATE: {
         const GdItem* g = (const GdItem*)item;
-        int R = gd_rows_per_tile(g->mx, g->my, kind == OP_GD_PROJECT ? GD_TILE_PROJ : GD_TILE);
+        int R = gd_rows_per_tile(g->mx, g->my, gd_tile(kind));
         return (g->my + R - 1) / R;
     }
     case OP_GD_MOVES: case OP_GD_DIAGRES: return ngroups_elem(((const GdItem*)item)->n);
@@ -3971,9 +4154,9 @@ void launch_op(int kind, const void* d_items, const int* d_gstart, int nitems, i
     case OP_GSB_SETUP: hipLaunchKernelGGL(k_gsb_setup, ge, dim3(GSB_THREADS), 0, s, (const GsbItem*)d_items, d_gstart, nitems, ro); break;
     case OP_GSB_WALK: hipLaunchKernelGGL(k_gsb_walk, ge, dim3(GSB_THREADS), lds_bytes, s, (const GsbItem*)d_items, d_gstart, nitems, ro); break;
     case OP_GSB_CHECK: hipLaunchKernelGGL(k_gsb_check, ge, dim3(GSB_THREADS), 0, s, (const GsbItem*)d_items, d_gstart, nitems, ro); break;
-    case OP_GD_PROJECT: hipLaunchKernelGGL(k_gd_project, ge, dim3(GD_THREADS), lds_bytes, s, (const GdItem*)d_items, d_gstart, nitems, ro); break;
+    case OP_GD_PROJECT: hipLaunchKernelGGL(k_gd_project, ge, dim3(GD_ROW_THREADS), lds_bytes, s, (const GdItem*)d_items, d_gstart, nitems, ro); break;
     case OP_GD_PROBE: hipLaunchKernelGGL(k_gd_probe, ge, dim3(GD_THREADS), lds_bytes, s, (const GdItem*)d_items, d_gstart, nitems, ro); break;
-    case OP_GD_UPDATE: hipLaunchKernelGGL(k_gd_update, ge, dim3(GD_THREADS), lds_bytes, s, (const GdItem*)d_items, d_gstart, nitems, ro); break;
+    case OP_GD_UPDATE: hipLaunchKernelGGL(k_gd_update, ge, dim3(GD_ROW_THREADS), lds_bytes, s, (const GdItem*)d_items, d_gstart, nitems, ro); break;
     case OP_GD_MOVES: hipLaunchKernelGGL(k_gd_moves, ge, te, 0, s, (const GdItem*)d_items, d_gstart, nitems, ro); break;
     case OP_GD_DIAGRES: hipLaunchKernelGGL(k_gd_diagres, ge, te, 0, s, (const GdItem*)d_items, d_gstart, nitems, ro); break;
     case OP_SETUP: hipLaunchKernelGGL(k_setup, ge, te, 0, s, (const SetupItem*)d_items, d_gstart, nitems, ro); break;
@@ -4093,9 +4276,9 @@ size_t op_lds(int kind, const void* item, int stage)
     if (kind == OP_GSB_WALK) return gsb_lds(((const GsbItem*)item)->mx);
     if (kind == OP_GD_PROJECT || kind == OP_GD_PROBE || kind == OP_GD_UPDATE) {
         const GdItem* g = (const GdItem*)item;
-        int R = gd_rows_per_tile(g->mx, g->my, kind == OP_GD_PROJECT ? GD_TILE_PROJ : GD_TILE);
+        int R = gd_rows_per_tile(g->mx, g->my, gd_tile(kind));
         size_t cells = (size_t)R * gd_row_stride(g->mx);
-        return cells * ((kind == OP_GD_PROJECT ? 7 : 3) * sizeof(double) + 1) + 16;
+        return cells * (4 * sizeof(double) + (kind == OP_GD_PROJECT ? 1 : 0)) + 16;
     }
     if (kind == OP_STDYGS) {
         const GsItem* g = (const GsItem*)item;
