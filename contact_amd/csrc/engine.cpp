@@ -608,8 +608,8 @@ private:
     // the last block), and the convergence test.  complete_async advances it each time the
     // step's event has completed; patches that have converged leave the later sweeps.
     struct GsbGroup {
-        int B = 8;                            // rows per block
         std::vector<GsItem> gs;
+        std::vector<int> B;                   // rows per block of each patch
         std::vector<int> first, last, nb;     // interior rows and blocks per patch
         std::vector<char> active;
         std::vector<std::array<double, 10>> fin;
@@ -655,13 +655,13 @@ private:
     {
         const int nitems = (int)reqs.size(), K = 10;
         auto G = std::make_shared<GsbGroup>();
-        if (const char* e = std::getenv("CNTC_GSB_ROWS"); e && std::atoi(e) > 0) G->B = std::atoi(e);
-        int mymax = 0;
+        int rows = 1 << 30, nbb = 0;
+        if (const char* e = std::getenv("CNTC_GSB_ROWS"); e && std::atoi(e) > 0) rows = std::atoi(e);
         for (auto* r : reqs) {
             G->gs.push_back(r->item.gs);
-            mymax = std::max(mymax, r->item.gs.my);
+            G->B.push_back(std::max(1, std::min(rows, gsb_block_rows(r->item.gs.mx))));
+            nbb = std::max(nbb, (r->item.gs.my + G->B.back() - 1) / G->B.back());
         }
-        const int nbb = (mymax + G->B - 1) / G->B;
         const size_t isz = std::max(sizeof(ConvItem), sizeof(GsbItem));
         const size_t one = align256(isz * nitems) + 3 * align256(sizeof(int) * (nitems + 1));
         G->cap_sw = (size_t)(2 * nbb + 2) * one;
@@ -774,13 +774,13 @@ private:
                 const int i = G.act[a];
                 if (G.nb[i] <= b) continue;
                 GsbItem w = gsb_item(G.gs[i], 1, st_of(i));
-                w.y0 = G.first[i] + b * G.B;
-                w.y1 = std::min(G.last[i] + 1, w.y0 + G.B);
+                w.y0 = G.first[i] + b * G.B[i];
+                w.y1 = std::min(G.last[i] + 1, w.y0 + G.B[i]);
                 // d of the previous block (for the first block: the last block of the sweep
                 // before, whose change no product used)
                 const int pb = b > 0 ? b - 1 : G.nb[i] - 1;
-                w.z0 = G.first[i] + pb * G.B;
-                w.z1 = std::min(G.last[i] + 1, w.z0 + G.B);
+                w.z0 = G.first[i] + pb * G.B[i];
+                w.z1 = std::min(G.last[i] + 1, w.z0 + G.B[i]);
                 who.push_back(i);
                 its.push_back(w);
                 if (G.nb[i] > b + 1) whoc.push_back(i);
@@ -825,7 +825,7 @@ private:
                 if (std::isfinite(f) && std::isfinite(l) && l >= f) {
                     G.first[i] = (int)f;
                     G.last[i] = (int)l;
-                    G.nb[i] = (G.last[i] - G.first[i]) / G.B + 1;
+                    G.nb[i] = (G.last[i] - G.first[i]) / G.B[i] + 1;
                 }
                 G.nbmax = std::max(G.nbmax, G.nb[i]);
                 G.act.push_back(i);

@@ -2860,7 +2860,6 @@ struct GsRow {
     double* pn;
     double* wx; double* wy;       // ws
     double* ucx; double* ucy;     // influence of other rows, unscaled (times ga_inv)
-    const double* zx; const double* zy;   // influence of other rows, scaled (null: none)
     const double* stc;            // own-row coefficients, 4 blocks of 2 mx (offsets q - mx)
     int8_t* el;
 };
@@ -2892,8 +2891,7 @@ __device__ inline double wave_sum(double v)
 // Called by all 64 lanes of wavefront 0.
 __device__ void gs_walk_span(const GsRow& R, int mx, int j0, int j1, size_t r0, int& ixw, int iend,
                              int& lastna, double& difacc, double ga_inv, double eps, double mu,
-                             double omegah, double omegas, double* gsx, double* gsy,
-                             bool s_lds = false)
+                             double omegah, double omegas, double* gsx, double* gsy)
 {
     const int lane = threadIdx.x, M2 = 2 * mx;
     for (; ixw < iend; ixw++) {
@@ -2923,13 +2921,8 @@ __device__ void gs_walk_span(const GsRow& R, int mx, int j0, int j1, size_t r0, 
             double a21 = ga_inv * (R.stc[2 * M2 + b0] - R.stc[2 * M2 + bj]);
             double a22 = ga_inv * (R.stc[3 * M2 + b0] - R.stc[3 * M2 + bj]);
             double sv[2];
-            if (R.zx) {
-                sv[0] = (R.wx[ix] + R.zx[ix]) + ga_inv * (R.ucx[ix] + qsx);
-                sv[1] = (R.wy[ix] + R.zy[ix]) + ga_inv * (R.ucy[ix] + qsy);
-            } else {
-                sv[0] = R.wx[ix] + ga_inv * (R.ucx[ix] + qsx);
-                sv[1] = R.wy[ix] + ga_inv * (R.ucy[ix] + qsy);
-            }
+            sv[0] = R.wx[ix] + ga_inv * (R.ucx[ix] + qsx);
+            sv[1] = R.wy[ix] + ga_inv * (R.ucy[ix] + qsy);
             const double opx = R.px[ix], opy = R.py[ix];
             double pr[3] = {opx, opy, R.pn[ix]};
             int8_t e8 = R.el[ix];
@@ -2944,15 +2937,8 @@ __device__ void gs_walk_span(const GsRow& R, int mx, int j0, int j1, size_t r0, 
                 R.px[ix] = pr[0];
                 R.py[ix] = pr[1];
                 R.el[ix] = e8;
-                if (s_lds) {
-                    // kept in LDS in place of this element's other-row influence (read once,
-                    // above) and stored with the row: no global store on the element chain
-                    R.ucx[ix] = sv[0];
-                    R.ucy[ix] = sv[1];
-                } else {
-                    gsx[ii] = sv[0];
-                    gsy[ii] = sv[1];
-                }
+                gsx[ii] = sv[0];
+                gsy[ii] = sv[1];
             }
         }
         __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
@@ -3116,7 +3102,7 @@ __global__ void __launch_bounds__(GS_THREADS) k_stdygs3(const GsItem* __restrict
     int8_t* rel = (int8_t*)(ri1 + my);
     double* stg = gs_lds + gs3_stage_off(mx, my) / 8;
     const int SW = gs3_stage_stride(mx);
-    const GsRow R{rpx, rpy, rdpx, rdpy, rg, rpn, rwx, rwy, ucx, ucy, nullptr, nullptr, stc, rel};
+    const GsRow R{rpx, rpy, rdpx, rdpy, rg, rpn, rwx, rwy, ucx, ucy, stc, rel};
     double* dpx = I.dpx;
     double* dpy = I.dpy;
     // the xx, xy and yy coefficient blocks: the coefficient kernel writes the xy and yx blocks
@@ -3477,22 +3463,339 @@ __global__ void __launch_bounds__(GSB_THREADS) k_gsb_setup(const GsbItem* __rest
     }
 }
 
-// LDS of k_gsb_walk: 14 row arrays, the own-row coefficients (4 x 2 mx), the staging of a
-// row product (3 coefficient windows and 2 source rows), the states of the row
-__host__ __device__ inline int gsb_window(int mx) { return (2 * mx + GS3_TB + GS3_QB + 3) / 4 * 4; }
-__host__ __device__ inline size_t gsb_lds(int mx)
+// LDS of k_gsb_walk for blocks of `rows` rows: the coefficient rows of the offsets 0 (xx, yy) and
+// 1 .. rows - 1 (xx, xy = yx, yy), each 2 mx; two sets of row elements with their differences at
+// the row's start; and with more than one row the changes of the rows walked and their influence
+// on the next row (two sets, and the four parts of the last row's).
+__host__ __device__ inline size_t gsb_lds_rows(int mx, int rows)
 {
-    return ((size_t)14 * mx + 8 * mx + 3 * gsb_window(mx) + 2 * (mx + GS3_QB) + 2 * GSB_THREADS) *
-               sizeof(double) + mx + 64;
+    return ((size_t)(4 + 6 * (rows - 1) + 20) + (rows > 1 ? 2 * rows + 12 : 0)) * mx * sizeof(double) +
+           (size_t)4 * rows * sizeof(int) + 64;
+}
+constexpr int GSB_MAX_ROWS = 8;
+// Rows per block: as many as fit the LDS beside the kernel's static part (0: not even one).  More
+// rows mean fewer products of the whole grid per sweep; those a block holds are summed from LDS.
+__host__ __device__ inline int gsb_fit_rows(int mx)
+{
+    int r = GSB_MAX_ROWS;
+    while (r > 0 && gsb_lds_rows(mx, r) + 2048 > MAX_LDS) r--;
+    return r;
 }
 
-// The walk of one block of rows.  For row t of the block, the influence of every other row is
-//   z_t - A(0) dp_t + sum over the block's rows j < t of A(t - j) d_j
-// (z = A dp at the block's start includes row t itself and the block's rows at their
-// start values; d_j = the change of row j's differences in this block), then wavefront 0
-// walks the row with the own-row influence of the current differences, as k_stdygs3 does.
-// The row products run on all threads: a thread owns GS3_TB consecutive targets and takes
-// the sources in chunks of GS3_QB from one coefficient window per block (xx, xy = yx, yy).
+// an element of the row being walked (LDS)
+struct GsbEl {
+    double px, py;      // p
+    double g, e;        // bound mu pn, state
+    double dx, dy;      // difference along x
+    double ux, uy;      // s without the row's own changes; s itself once the element is solved
+};
+
+// v of slot `q` (wavefront-uniform) of a register array, lane `l`
+template <int NS>
+__device__ inline double slot_lane(const double (&v)[NS], int q, int l)
+{
+    double r = v[0];
+#pragma unroll
+    for (int s = 1; s < NS; s++)
+        if (q == s) r = v[s];
+    return lane_f64(r, l);
+}
+__device__ inline bool uniform_any(bool c) { return __builtin_amdgcn_ballot_w64(c) != 0; }
+// keeps what follows from x in the branch it is written in (loop-invariant code motion would
+// form every branch's values on the way in)
+__device__ inline double stay_here(double x)
+{
+    asm volatile("" : "+v"(x));
+    return x;
+}
+
+// elmtrc (src/m_solvpt.f90:3258-3807) on the latency path: the steps of elmtrc with scale_dir,
+// on data that every lane holds alike, so that its branches are scalar.  c12 = c21 = 0: within a
+// row the xy coefficients vanish by symmetry (the tables hold their rounding, 1e-17 of xx).  The
+// iterates are those of elmtrc: the Newton corrections divide through a once refined reciprocal
+// (good to 2^-45 of a correction), the starting direction through a once refined reciprocal
+// square root.
+__device__ inline void elmtrc_uniform(int& el, double c11, double c22, double eps, double& p0, double& p1,
+                                      double tb, double& s0, double& s1, double omegah, double omegas)
+{
+    const int maxnr = 10;
+    const double prc = 0.0001, PI = 3.14159265358979323846;
+    const double o0 = p0, o1 = p1, in0 = s0, in1 = s1;
+    const double si0x = fma(-c11, o0, in0), si0y = fma(-c22, o1, in1);
+    double six = 0.0, siy = 0.0;
+    bool violat = true;
+    for (int itry = 1; itry <= 4 && violat; itry++) {
+        if (el == ADHES) {
+            const double d0 = -in0 * fast_rcp(stay_here(c11)), d1 = -in1 * fast_rcp(stay_here(c22));
+            p0 = fma(omegah, d0, o0);
+            p1 = fma(omegah, d1, o1);
+            const double p2 = fma(p0, p0, p1 * p1), bnd = fmin(tb, 1e20), b2 = bnd * bnd;
+            violat = false;
+            if (uniform_any(!(p2 <= b2))) {
+                const double q0 = o0 + d0, q1 = o1 + d1;
+                if (uniform_any(fma(q0, q0, q1 * q1) <= b2)) {
+                    const double f = bnd * fast_rsqrt(p2);
+                    p0 *= f;
+                    p1 *= f;
+                } else {
+                    violat = true;
+                }
+            }
+            six = fma(c11, p0, si0x);
+            siy = fma(c22, p1, si0y);
+        } else if (el == SLIP) {
+            const double bx = stay_here(si0x), by = stay_here(si0y);
+            const double a2 = fma(bx, bx, by * by), y = __builtin_amdgcn_rsq(a2);
+            const double f = -tb * fma(y, fma(-0.5 * a2 * y, y, 0.5), y);
+            p0 = f * bx;
+            p1 = f * by;
+            const double tb2 = tb * tb, dc = c11 - c22, lim = prc * eps * tb;
+            six = fma(c11, p0, bx);
+            siy = fma(c22, p1, by);
+            double fk0 = fma(p1, six, -(p0 * siy)), fk1 = fma(p0, p0, fma(p1, p1, -tb2));
+            for (int itnr = 1;; itnr++) {
+                const double g00 = fma(dc, p1, -by), g01 = fma(dc, p0, bx);
+                const double g10 = 2.0 * p0, g11 = 2.0 * p1;
+                const double det = fma(g00, g11, -(g01 * g10));
+                const double n0 = fma(g01, fk1, -(g11 * fk0)), n1 = fma(g10, fk0, -(g00 * fk1));
+                double r = __builtin_amdgcn_rcp(det);
+                r = fma(r, fma(-det, r, 1.0), r);
+                r = det == 0.0 ? 0.0 : r;      // (no correction then, as in elmtrc)
+                p0 = fma(n0, r, p0);
+                p1 = fma(n1, r, p1);
+                six = fma(c11, p0, bx);
+                siy = fma(c22, p1, by);
+                fk0 = fma(p1, six, -(p0 * siy));
+                fk1 = fma(p0, p0, fma(p1, p1, -tb2));
+                if (!uniform_any(fabs(fk0) + fabs(fk1) >= lim)) break;
+                if (itnr >= maxnr) break;
+            }
+            if (omegas == 1.0) {
+                const double p2 = fma(p0, p0, p1 * p1);
+                const double h = tb * fast_rsqrt(p2);
+                p0 = p2 > 0.0 ? p0 * h : tb;
+                p1 = p2 > 0.0 ? p1 * h : 0.0;
+            } else {
+                const double alph0 = atan2(stay_here(o1), stay_here(o0)), alph1 = atan2(p1, p0);
+                double dalph = alph1 - alph0;
+                if (dalph < -PI) dalph += 2.0 * PI;
+                if (dalph > PI) dalph -= 2.0 * PI;
+                const double alph = alph0 + omegas * dalph;
+                p0 = tb * cos(alph);
+                p1 = tb * sin(alph);
+            }
+            violat = uniform_any(fabs(p0) > fabs(p1) ? p0 * six > 0.0 : p1 * siy > 0.0);
+        }
+        if (itry <= 3 && violat) el = el == ADHES ? SLIP : (el == SLIP ? PLAST : ADHES);
+    }
+    s0 = six;
+    s1 = siy;
+}
+
+// Wavefront 0's walk along the interior elements t0 .. t1 of a row (src/m_solvpt.f90:2950-3127),
+// each element's 2x2 problem in order from the trailing edge, then the rebuild of the upstream
+// part of the row.  The time of an element is a chain of dependent operations, so as little as
+// possible is on it:
+//   - u, the shift at every element of the row, and p are in registers (slot s of lane l holds
+//     element t0 + 64 s + l).  A solved element changes its difference by D and that of the
+//     first upstream element not in adhesion, la, by -D (the adhesion elements between move
+//     along: p by D, differences unchanged), so that u += (A(. - ix) - A(. - la)) D for the
+//     elements ahead; no sum over the row is formed.
+//   - the next element's data and coefficients are read from LDS while this one is solved.
+//   - every lane solves the element on the same data (scalar branches, elmtrc_uniform).
+// An adhesion element upstream that the move takes over its bound is clipped and the elements
+// below it move by its change: one more term of u for each (rare).
+// tab: own-row coefficients (xx, yy) times 1/G, offsets q - mx.
+template <int NS>
+__device__ __forceinline__ void gsb_walk_row(GsbEl* const row, const double* early, const double* part, int mx,
+                                             int t0, int t1, const GdCell* const tab, double& difacc,
+                                             double eps, double omegah, double omegas)
+{
+    const int lane = threadIdx.x & 63;
+    // rows of more than 256 elements read coefficients and bounds where they are used: 14 slots of
+    // them do not fit the registers
+    constexpr bool KEEP = NS <= 4;
+    constexpr int NK = KEEP ? NS : 1;
+    double Ux[NS], Uy[NS], Px[NS], Py[NS];
+    double G2[NK];                           // bounds squared
+    GdCell c[NK], l[NK];                     // A(k - ix), A(k - la)
+    const GdCell* tk[NS];                    // A(k - 0) of this lane's elements
+    auto elem = [&](int s) { return t0 + 64 * s + lane; };
+    // (the trailing-edge column has no contact: ConvexGS solves those cases)
+    int la = t0 - 1 >= 0 ? t0 - 1 : 0;
+#pragma unroll
+    for (int s = 0; s < NS; s++) {
+        const int k = elem(s), kc = k <= t1 ? k : t1;
+        double ux = row[kc].ux, uy = row[kc].uy;
+        if (early) {
+            ux += early[kc];
+            uy += early[mx + kc];
+            for (int q = 0; q < 4; q++) {
+                ux += part[2 * q * mx + kc];
+                uy += part[(2 * q + 1) * mx + kc];
+            }
+        }
+        Ux[s] = ux;
+        Uy[s] = uy;
+        Px[s] = row[kc].px;
+        Py[s] = row[kc].py;
+        tk[s] = tab + kc + mx;
+        if constexpr (KEEP) {
+            G2[s] = row[kc].g * row[kc].g;
+            c[s] = tk[s][-t0];
+            l[s] = tk[s][-la];
+        }
+    }
+    const GdCell b0 = tab[mx], b1 = tab[mx - 1];
+    // p of element la (0 in the exterior) and of la + 1
+    double plax = 0.0, play = 0.0, pnex = 0.0, pney = 0.0;
+    // the element being solved, and A(la - ix)
+    GsbEl E = row[t0];
+    GdCell a = b1;
+    double dif = 0.0;
+    for (int ix = t0; ix <= t1; ix++) {
+        // reads for the next element, on their way while this one is solved
+        const int nx = ix < t1 ? ix + 1 : ix;
+        GsbEl N;
+        N.px = row[nx].px; N.py = row[nx].py; N.g = row[nx].g; N.e = row[nx].e; N.dx = row[nx].dx; N.dy = row[nx].dy;
+        const GdCell na = tab[la - nx + mx];
+        GdCell nc[NK];
+        if constexpr (KEEP)
+#pragma unroll
+            for (int s = 0; s < NS; s++) nc[s] = tk[s][-nx];
+        int e = __builtin_amdgcn_readfirstlane((int)E.e);
+        if (e >= ADHES) {
+            const int q = (ix - t0) >> 6, ol = (ix - t0) & 63;
+            const bool near_la = la == ix - 1;
+            double s0 = slot_lane<NS>(Ux, q, ol), s1 = slot_lane<NS>(Uy, q, ol);
+            double p0 = E.px, p1 = E.py;
+            elmtrc_uniform(e, b0.x - a.x, b0.y - a.y, eps, p0, p1, E.g, s0, s1, omegah, omegas);
+            const double Dx = p0 - E.px, Dy = p1 - E.py;
+            dif += Dx * Dx + Dy * Dy;
+#pragma unroll
+            for (int s = 0; s < NS; s++) {
+                GdCell ca, cl;
+                if constexpr (KEEP) {
+                    ca = c[s];
+                    cl = l[s];
+                } else {
+                    ca = tk[s][-ix];
+                    cl = tk[s][-la];
+                }
+                Ux[s] = fma(ca.x - cl.x, Dx, Ux[s]);
+                Uy[s] = fma(ca.y - cl.y, Dy, Uy[s]);
+                const bool own = elem(s) == ix;
+                Px[s] = own ? p0 : Px[s];
+                Py[s] = own ? p1 : Py[s];
+            }
+            if (near_la) {
+                pnex = p0;
+                pney = p1;
+            } else {
+                // the adhesion elements between la and ix move by D
+                double Mx = Dx, My = Dy;
+                int hi = ix;
+                for (;;) {
+                    int f = la;              // the first element over its bound, from ix; la: none
+#pragma unroll
+                    for (int s = 0; s < NS; s++) {
+                        double g2;
+                        if constexpr (KEEP) {
+                            g2 = G2[s];
+                        } else {
+                            const double g = row[elem(s) <= t1 ? elem(s) : t1].g;
+                            g2 = g * g;
+                        }
+                        const double qx = Px[s] + Mx, qy = Py[s] + My;
+                        const unsigned long long over = __builtin_amdgcn_ballot_w64(
+                            elem(s) > la && elem(s) < hi && fma(qx, qx, qy * qy) > g2);
+                        if (over) f = t0 + 64 * s + 63 - __clzll((long long)over);
+                    }
+#pragma unroll
+                    for (int s = 0; s < NS; s++) {
+                        const bool go = elem(s) > f && elem(s) < hi;
+                        Px[s] = go ? Px[s] + Mx : Px[s];
+                        Py[s] = go ? Py[s] + My : Py[s];
+                    }
+                    if (f == la) break;
+                    const int fq = (f - t0) >> 6, fl = (f - t0) & 63;
+                    const double ox = slot_lane<NS>(Px, fq, fl), oy = slot_lane<NS>(Py, fq, fl);
+                    const double wx = ox + Mx, wy = oy + My;
+                    const double fa = row[f].g / sqrt(wx * wx + wy * wy);
+                    const double vx = wx * fa, vy = wy * fa;
+                    // p(f + 1), already moved
+                    const int uq = (f + 1 - t0) >> 6, ul = (f + 1 - t0) & 63;
+                    const double upx = slot_lane<NS>(Px, uq, ul), upy = slot_lane<NS>(Py, uq, ul);
+                    if (lane == 0) {
+                        row[f].dx = vx - upx;
+                        row[f].dy = vy - upy;
+                    }
+                    const double nMx = vx - ox, nMy = vy - oy;
+#pragma unroll
+                    for (int s = 0; s < NS; s++) {
+                        const GdCell cf = tk[s][-f], cl = tk[s][-la];
+                        Ux[s] = fma(cf.x - cl.x, nMx - Mx, Ux[s]);
+                        Uy[s] = fma(cf.y - cl.y, nMy - My, Uy[s]);
+                        const bool own = elem(s) == f;
+                        Px[s] = own ? vx : Px[s];
+                        Py[s] = own ? vy : Py[s];
+                    }
+                    Mx = nMx;
+                    My = nMy;
+                    hi = f;
+                }
+                const int uq = (la + 1 - t0) >> 6, ul = (la + 1 - t0) & 63;
+                pnex = slot_lane<NS>(Px, uq, ul);
+                pney = slot_lane<NS>(Py, uq, ul);
+            }
+            if (lane == 0) {
+                row[la].dx = plax - pnex;
+                row[la].dy = play - pney;
+                row[ix].e = (double)e;
+                row[ix].dx = E.dx + Dx;
+                row[ix].dy = E.dy + Dy;
+                row[ix].ux = s0;
+                row[ix].uy = s1;
+            }
+            plax = e != ADHES ? p0 : plax;
+            play = e != ADHES ? p1 : play;
+        } else {
+            plax = 0.0;
+            play = 0.0;
+        }
+        a = na;
+        if (e != ADHES) {
+            la = ix;
+            a = b1;
+            if constexpr (KEEP)
+#pragma unroll
+                for (int s = 0; s < NS; s++) l[s] = c[s];
+        }
+        E.px = N.px; E.py = N.py; E.g = N.g; E.e = N.e; E.dx = N.dx; E.dy = N.dy;
+        if constexpr (KEEP)
+#pragma unroll
+            for (int s = 0; s < NS; s++) c[s] = nc[s];
+    }
+    difacc += dif;
+#pragma unroll
+    for (int s = 0; s < NS; s++)
+        if (elem(s) <= t1) {
+            row[elem(s)].px = Px[s];
+            row[elem(s)].py = Py[s];
+        }
+}
+
+// The walk of one block of rows.  For row t of the block, the influence of every other row and
+// of the row itself at its start is
+//   z_t + sum over the block's rows j < t of A(t - j) d_j
+// (z = A dp at the block's start; d_j = the change of row j's differences in this block), to
+// which wavefront 0 adds the row's own changes as it walks (gsb_walk_row).  Meanwhile the other
+// wavefronts read the next row and sum the influence on it of the rows walked before this one;
+// what this row's own change adds to it is summed by all four after the walk.  The block's
+// coefficient rows stay in LDS.  Latency-bound: one wavefront's chain.  With the sum over the row
+// formed for each element, and every row pair's coefficients staged from memory in the gap
+// between two rows, a block of eight rows of a 151 x 97 patch took 1515 us (2.1 us an element),
+// 589 us so; a sweep of an 11 x 11 patch 310 us, 52 us so.
 __global__ void __launch_bounds__(GSB_THREADS) k_gsb_walk(const GsbItem* __restrict__ items, const int* __restrict__ gstart,
                                                           int nitems, RedOut ro)
 {
@@ -3500,199 +3803,143 @@ __global__ void __launch_bounds__(GSB_THREADS) k_gsb_walk(const GsbItem* __restr
     (void)ro;
     int it = find_item(gstart, nitems, blockIdx.x);
     const GsbItem& I = items[it];
-    const int mx = I.mx, my = I.my, tid = threadIdx.x, T = blockDim.x, M2 = 2 * mx;
-    double* rpx = gsb_lds_;
-    double* rpy = rpx + mx;
-    double* rdpx = rpy + mx;
-    double* rdpy = rdpx + mx;
-    double* r0x = rdpy + mx;               // differences at the row's start
-    double* r0y = r0x + mx;
-    double* rg = r0y + mx;
-    double* rpn = rg + mx;
-    double* rwx = rpn + mx;
-    double* rwy = rwx + mx;
-    double* ucx = rwy + mx;
-    double* ucy = ucx + mx;
-    double* rzx = ucy + mx;
-    double* rzy = rzx + mx;
-    double* stc = rzy + mx;                // own-row coefficients, offsets (q - mx, 0)
-    double* sc = stc + 4 * M2;             // product staging: 3 windows, then 2 source rows
-    double* red = sc + 3 * gsb_window(mx) + 2 * (mx + GS3_QB);
-    int8_t* rel = (int8_t*)(red + 2 * GSB_THREADS);
-    const int* rj0 = I.rng;
-    const int* rj1 = rj0 + my;
-    const int* ri0 = rj1 + my;
-    const int* ri1 = ri0 + my;
-    const double* cfs[3] = {I.cf[0][0], I.cf[0][1], I.cf[1][1]};   // yx = xy
-    const double* cfb[4] = {I.cf[0][0], I.cf[0][1], I.cf[1][0], I.cf[1][1]};
-    const GsRow R{rpx, rpy, rdpx, rdpy, rg, rpn, rwx, rwy, ucx, ucy, rzx, rzy, stc, rel};
+    const int mx = I.mx, my = I.my, tid = threadIdx.x, T = blockDim.x, M2 = 2 * mx, wave = tid >> 6;
+    const int y0 = I.y0, B = I.y1 - I.y0;
+    GdCell* const tab0 = (GdCell*)gsb_lds_;              // offset 0: (xx, yy)[2 mx], times 1/G
+    double* const tab = gsb_lds_ + 4 * mx;               // [offset - 1][xx, xy, yy][2 mx], times 1/G
+    GsbEl* const els = (GsbEl*)(tab + (size_t)6 * (B - 1) * mx);   // two sets of row elements
+    double* const r0 = (double*)(els + 2 * mx);          // two sets [x, y][mx]: differences at the start
+    double* const dd = r0 + 4 * mx;                      // [row][x, y][mx]: changes of the walked rows
+    double* const early = dd + (B > 1 ? 2 * B * mx : 0); // two sets [x, y][mx]: influence of earlier rows
+    double* const part = early + 4 * mx;                 // four parts [x, y][mx]: of the last row
+    int* const rg = (int*)(early + (B > 1 ? 12 * mx : 0)); // [row][first, last source; first, last interior]
+    // row t into set b, by threads `first`, first + 1, ...
+    auto load_row = [&](int t, int b, int first) {
+        const size_t o = (size_t)t * mx;
+        for (int ix = tid - first; ix < mx; ix += T - first) {
+            GsbEl E;
+            E.px = as_global(I.px)[o + ix];
+            E.py = as_global(I.py)[o + ix];
+            E.dx = as_global(I.dpx)[o + ix];
+            E.dy = as_global(I.dpy)[o + ix];
+            const double pn = as_global(I.pn)[o + ix];
+            const double wx = as_global(I.wsx)[o + ix], wy = as_global(I.wsy)[o + ix];
+            const double zx = as_global(I.zx)[o + ix], zy = as_global(I.zy)[o + ix];
+            E.e = (double)as_global(I.el)[o + ix];
+            E.g = I.mu * pn;
+            E.ux = wx + zx;
+            E.uy = wy + zy;
+            els[b * mx + ix] = E;
+            r0[2 * b * mx + ix] = E.dx;
+            r0[(2 * b + 1) * mx + ix] = E.dy;
+        }
+    };
+    // (ax, ay) += the influence at element k of row n of the changes q0 <= q < q1 of row j
+    auto row_sum = [&](int k, int n, int j, int q0, int q1, double& ax, double& ay) {
+        const double* const xx = tab + (size_t)(n - j - 1) * 3 * M2 + k + mx;
+        const double *const xy = xx + M2, *const yy = xy + M2;
+        const double *const dx = dd + (size_t)2 * j * mx, *const dy = dx + mx;
+        double sx = 0.0, sy = 0.0;
+#pragma unroll 4
+        for (int q = q0; q < q1; q++) {
+            const double a = xy[-q], x = dx[q], y = dy[q];
+            sx = fma(xx[-q], x, fma(a, y, sx));
+            sy = fma(yy[-q], y, fma(a, x, sy));
+        }
+        ax += sx;
+        ay += sy;
+    };
 
     // d of the previous block has been used by its product: clear it
     for (size_t e = (size_t)I.z0 * mx + tid; e < (size_t)I.z1 * mx; e += T) {
-        I.ddx[e] = 0.0;
-        I.ddy[e] = 0.0;
+        as_global(I.ddx)[e] = 0.0;
+        as_global(I.ddy)[e] = 0.0;
     }
-    for (int e = tid; e < 4 * M2; e += T) {
-        const int b = e / M2, q = e - b * M2;
-        stc[e] = cfb[b][(size_t)my * M2 + q];
-    }
-    double difacc = 0.0, flops = 0.0;   // thread 0
-    double ax[GS3_TB], ay[GS3_TB];
-    // ax, ay (targets of row tr) += A(tr - sy) src over the source range [j0, j0 + nq), the
-    // source row given in global memory (sgx, sgy) or, for the row itself, in LDS negated
-    auto row_prod = [&](int tr, int sy, const double* sgx, const double* sgy, bool self) {
-        const int t0 = ri0[tr], nt = ri1[tr] - t0 + 1;
-        const int j0 = rj0[sy], nq = rj1[sy] - j0 + 1;
-        if (nq <= 0) return;
-        const int ntg = (nt + GS3_TB - 1) / GS3_TB, ntp = ntg * GS3_TB;
-        const int P = T / ntg > 0 ? T / ntg : 1;
-        const int tg = tid % ntg, part = tid / ntg;
-        const int Q = (nq + GS3_QB - 1) / GS3_QB * GS3_QB;
-        const int Wn = ntp + Q - 1, Wp = (Wn + 1 + 3) / 4 * 4;
-        // window S[k], k = t - q + Q - 1: coefficient of target t0 + t and source j0 + q
-        const int col0 = t0 - j0 - (Q - 1) + mx;
-        __syncthreads();
-#pragma unroll
-        for (int bb = 0; bb < 3; bb++) {
-            const double* crow = cfs[bb] + (size_t)(tr - sy + my) * M2;
-            for (int k = tid; k < Wp; k += T) {
-                const int col = col0 + k;
-                sc[bb * Wp + k] = (k < Wn && col >= 0 && col < M2) ? crow[col] : 0.0;
-            }
-        }
-        double* sdx = sc + 3 * Wp;
-        double* sdy = sdx + Q;
-        for (int e = tid; e < Q; e += T) {
-            const bool in = e < nq;
-            if (self) {
-                sdx[e] = in ? -r0x[j0 + e] : 0.0;
-                sdy[e] = in ? -r0y[j0 + e] : 0.0;
-            } else {
-                sdx[e] = in ? sgx[(size_t)sy * mx + j0 + e] : 0.0;
-                sdy[e] = in ? sgy[(size_t)sy * mx + j0 + e] : 0.0;
-            }
-        }
-        __syncthreads();
-        if (part < P) {
-            const int nch = Q / GS3_QB;
-            for (int c = part; c < nch; c += P) {
-                const int kmin = tg * GS3_TB - c * GS3_QB + (Q - GS3_QB);
-                double qx[GS3_QB], qy[GS3_QB];
-#pragma unroll
-                for (int j = 0; j < GS3_QB; j++) {
-                    qx[j] = sdx[c * GS3_QB + j];
-                    qy[j] = sdy[c * GS3_QB + j];
-                }
-                const double2* w0 = (const double2*)(sc + kmin);
-                const double2* w1 = (const double2*)(sc + Wp + kmin);
-                const double2* w3 = (const double2*)(sc + 2 * Wp + kmin);
-                double v0[GS3_TB + GS3_QB], v1[GS3_TB + GS3_QB], v3[GS3_TB + GS3_QB];
-#pragma unroll
-                for (int m = 0; m < (GS3_TB + GS3_QB) / 2; m++) {
-                    const double2 a = w0[m], b2 = w1[m], d = w3[m];
-                    v0[2 * m] = a.x;
-                    v0[2 * m + 1] = a.y;
-                    v1[2 * m] = b2.x;
-                    v1[2 * m + 1] = b2.y;
-                    v3[2 * m] = d.x;
-                    v3[2 * m + 1] = d.y;
-                }
-#pragma unroll
-                for (int i = 0; i < GS3_TB; i++) {
-                    double accx = ax[i], accy = ay[i];
-#pragma unroll
-                    for (int j = 0; j < GS3_QB; j++) {
-                        const int m = i + GS3_QB - 1 - j;
-                        accx += v0[m] * qx[j] + v1[m] * qy[j];
-                        accy += v1[m] * qx[j] + v3[m] * qy[j];
-                    }
-                    ax[i] = accx;
-                    ay[i] = accy;
-                }
-            }
-        }
-        if (tid == 0) flops += 8.0 * nt * nq;
+    for (int e = tid; e < 4 * B; e += T) rg[e] = I.rng[(size_t)(e & 3) * my + y0 + (e >> 2)];
+    const double* const cfs[3] = {I.cf[0][0], I.cf[0][1], I.cf[1][1]};   // yx = xy
+    for (int e = tid; e < M2; e += T)
+        tab0[e] = GdCell{I.ga_inv * as_global(cfs[0])[(size_t)my * M2 + e], I.ga_inv * as_global(cfs[2])[(size_t)my * M2 + e]};
+    for (int c = 0; c < 3; c++)
+        for (int e = tid; e < (B - 1) * M2; e += T)
+            tab[(size_t)(e / M2 * 3 + c) * M2 + e % M2] = I.ga_inv * as_global(cfs[c])[(size_t)(my + 1) * M2 + e];
+    __syncthreads();
+    // the next row with an interior element, or B
+    auto next_row = [&](int r) {
+        do r++;
+        while (r < B && rg[4 * r + 3] < rg[4 * r + 2]);
+        return __builtin_amdgcn_readfirstlane(r);
     };
-    // ucx, ucy over the interior of row tr = the sum of the parts' accumulators
-    auto reduce_parts = [&](int tr) {
-        const int t0 = ri0[tr], nt = ri1[tr] - t0 + 1;
-        const int ntg = (nt + GS3_TB - 1) / GS3_TB;
-        const int P = T / ntg > 0 ? T / ntg : 1;
-        const int tg = tid % ntg, part = tid / ntg;
-        __syncthreads();
-        for (int i = 0; i < GS3_TB; i++) {
-            if (part < P) {
-                red[2 * (part * ntg + tg)] = ax[i];
-                red[2 * (part * ntg + tg) + 1] = ay[i];
-            }
-            __syncthreads();
-            for (int g = tid; g < ntg; g += T) {
-                const int c = g * GS3_TB + i;
-                if (c < nt) {
-                    double sx = 0.0, sy = 0.0;
-                    for (int p = 0; p < P; p++) {
-                        sx += red[2 * (p * ntg + g)];
-                        sy += red[2 * (p * ntg + g) + 1];
-                    }
-                    ucx[t0 + c] = sx;
-                    ucy[t0 + c] = sy;
+    double difacc = 0.0, flops = 0.0;   // (wavefront 0)
+    int r = next_row(-1), b = 0;
+    bool first = true;
+    if (r < B) load_row(y0 + r, 0, 0);
+    __syncthreads();
+    while (r < B) {
+        const int n = next_row(r);
+        const int t0 = __builtin_amdgcn_readfirstlane(rg[4 * r + 2]), t1 = __builtin_amdgcn_readfirstlane(rg[4 * r + 3]);
+        GsbEl* const row = els + b * mx;
+        if (wave == 0) {
+            const int nt = t1 - t0 + 1;
+            const double* ev = first ? nullptr : early + 2 * b * mx;
+            if (nt <= 64) gsb_walk_row<1>(row, ev, part, mx, t0, t1, tab0, difacc, I.eps, I.omegah, I.omegas);
+            else if (nt <= 128) gsb_walk_row<2>(row, ev, part, mx, t0, t1, tab0, difacc, I.eps, I.omegah, I.omegas);
+            else if (nt <= 256) gsb_walk_row<4>(row, ev, part, mx, t0, t1, tab0, difacc, I.eps, I.omegah, I.omegas);
+            else gsb_walk_row<14>(row, ev, part, mx, t0, t1, tab0, difacc, I.eps, I.omegah, I.omegas);
+            flops += 4.0 * nt * nt;
+        } else if (n < B) {
+            load_row(y0 + n, b ^ 1, 64);
+            // the influence on row n of the rows walked before this one
+            double* const ev = early + 2 * (b ^ 1) * mx;
+            for (int k = rg[4 * n + 2] + tid - 64; k <= rg[4 * n + 3]; k += T - 64) {
+                double ax = 0.0, ay = 0.0;
+                for (int j = 0; j < r; j++) {
+                    if (rg[4 * j + 3] < rg[4 * j + 2]) continue;
+                    row_sum(k, n, j, rg[4 * j], rg[4 * j + 1] + 1, ax, ay);
                 }
+                ev[k] = ax;
+                ev[mx + k] = ay;
             }
-            __syncthreads();
-        }
-    };
-
-    for (int t = I.y0; t < I.y1; t++) {
-        if (ri1[t] < ri0[t]) continue;   // no interior element in this row
-        const size_t r0 = (size_t)t * mx;
-        __syncthreads();
-        for (int ix = tid; ix < mx; ix += T) {
-            rpx[ix] = I.px[r0 + ix];
-            rpy[ix] = I.py[r0 + ix];
-            const double dx = I.dpx[r0 + ix], dy = I.dpy[r0 + ix];
-            rdpx[ix] = dx;
-            rdpy[ix] = dy;
-            r0x[ix] = dx;
-            r0y[ix] = dy;
-            const double pn = I.pn[r0 + ix];
-            rpn[ix] = pn;
-            rg[ix] = I.mu * pn;
-            rwx[ix] = I.wsx[r0 + ix];
-            rwy[ix] = I.wsy[r0 + ix];
-            rzx[ix] = I.zx[r0 + ix];
-            rzy[ix] = I.zy[r0 + ix];
-            rel[ix] = I.el[r0 + ix];
-        }
-#pragma unroll
-        for (int i = 0; i < GS3_TB; i++) ax[i] = ay[i] = 0.0;
-        // minus the row's own influence at its start (z holds it), plus the changes of the
-        // block's rows already walked
-        row_prod(t, t, nullptr, nullptr, true);
-        for (int j = I.y0; j < t; j++)
-            if (rj1[j] >= rj0[j]) row_prod(t, j, I.ddx, I.ddy, false);
-        reduce_parts(t);
-        if (tid < 64) {
-            const int t0 = ri0[t], nt = ri1[t] - t0 + 1;
-            int lastna = t0 - 1 >= 1 ? t0 - 1 : 0;
-            int ixw = t0;
-            gs_walk_span(R, mx, rj0[t], rj1[t], r0, ixw, t0 + nt, lastna, difacc, I.ga_inv, I.eps,
-                         I.mu, I.omegah, I.omegas, I.sx, I.sy, true);
         }
         __syncthreads();
-        const int t1 = ri1[t];
+        // the row's results
+        const size_t o = (size_t)(y0 + r) * mx;
         for (int ix = tid; ix < mx; ix += T) {
-            if (ix >= ri0[t] && ix <= t1 && rel[ix] >= ADHES) {
-                I.sx[r0 + ix] = ucx[ix];
-                I.sy[r0 + ix] = ucy[ix];
+            const GsbEl E = row[ix];
+            if (ix >= t0 && ix <= t1 && E.e >= (double)ADHES) {
+                as_global(I.sx)[o + ix] = E.ux;
+                as_global(I.sy)[o + ix] = E.uy;
             }
-            I.px[r0 + ix] = rpx[ix];
-            I.py[r0 + ix] = rpy[ix];
-            I.dpx[r0 + ix] = rdpx[ix];
-            I.dpy[r0 + ix] = rdpy[ix];
-            I.ddx[r0 + ix] = rdpx[ix] - r0x[ix];
-            I.ddy[r0 + ix] = rdpy[ix] - r0y[ix];
-            I.el[r0 + ix] = rel[ix];
+            const double cx = E.dx - r0[2 * b * mx + ix], cy = E.dy - r0[(2 * b + 1) * mx + ix];
+            as_global(I.px)[o + ix] = E.px;
+            as_global(I.py)[o + ix] = E.py;
+            as_global(I.dpx)[o + ix] = E.dx;
+            as_global(I.dpy)[o + ix] = E.dy;
+            as_global(I.ddx)[o + ix] = cx;
+            as_global(I.ddy)[o + ix] = cy;
+            as_global(I.el)[o + ix] = (int8_t)E.e;
+            if (B > 1) {
+                dd[(size_t)2 * r * mx + ix] = cx;
+                dd[(size_t)(2 * r + 1) * mx + ix] = cy;
+            }
         }
+        if (n >= B) break;
+        __syncthreads();
+        // the influence on row n of this row's change, a part of the sum by each wavefront
+        {
+            const int q0 = rg[4 * r], nq = rg[4 * r + 1] + 1 - q0, per = (nq + 3) / 4;
+            const int qa = q0 + min(nq, wave * per), qb = q0 + min(nq, (wave + 1) * per);
+            for (int k = rg[4 * n + 2] + (tid & 63); k <= rg[4 * n + 3]; k += 64) {
+                double ax = 0.0, ay = 0.0;
+                row_sum(k, n, r, qa, qb, ax, ay);
+                part[2 * wave * mx + k] = ax;
+                part[(2 * wave + 1) * mx + k] = ay;
+            }
+            if (tid == 0) flops += 8.0 * nq * (rg[4 * n + 3] - rg[4 * n + 2] + 1) * (r + 1);
+        }
+        __syncthreads();
+        r = n;
+        b ^= 1;
+        first = false;
     }
     if (tid == 0) {
         I.st[0] += difacc;
@@ -4273,7 +4520,7 @@ double op_bytes(int kind, const void* item, int stage)
 size_t op_lds(int kind, const void* item, int stage)
 {
     if (kind == OP_CONV || kind == OP_CONV32) return conv_lds(kind, (const ConvItem*)item, stage);
-    if (kind == OP_GSB_WALK) return gsb_lds(((const GsbItem*)item)->mx);
+    if (kind == OP_GSB_WALK) return gsb_lds_rows(((const GsbItem*)item)->mx, ((const GsbItem*)item)->y1 - ((const GsbItem*)item)->y0);
     if (kind == OP_GD_PROJECT || kind == OP_GD_PROBE || kind == OP_GD_UPDATE) {
         const GdItem* g = (const GdItem*)item;
         int R = gd_rows_per_tile(g->mx, g->my, gd_tile(kind));
@@ -4282,7 +4529,7 @@ size_t op_lds(int kind, const void* item, int stage)
     }
     if (kind == OP_STDYGS) {
         const GsItem* g = (const GsItem*)item;
-        if (stage == 3) return g->mx >= 2 ? gsb_lds(g->mx) : MAX_LDS + 1;   // rng needs 4 my <= 2 n
+        if (stage == 3) return g->mx >= 2 ? gsb_lds_rows(g->mx, 1) : MAX_LDS + 1;   // rng needs 4 my <= 2 n
         if (stage == 2) return gs3_lds(g->mx, g->my);
         if (stage == 1) return gs2_lds(g->mx, g->my);
         return (size_t)g->mx * (5 * sizeof(double) + 1) + (size_t)(2 * g->my + 1) * sizeof(int) + 16;
@@ -4303,6 +4550,8 @@ void launch_fill_u32(unsigned* p, size_t n, unsigned v, hipStream_t s)
     if (g > 1024) g = 1024;
     hipLaunchKernelGGL(k_fill_u32, dim3((unsigned)g), dim3(256), 0, s, p, n, v);
 }
+
+int gsb_block_rows(int mx) { return gsb_fit_rows(mx); }
 
 void conv_default_shape(const ConvItem* c, int* rpg, int* cpg)
 {

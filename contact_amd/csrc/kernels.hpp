@@ -28,6 +28,8 @@ size_t op_lds(int kind, const void* item, int stage);
 void launch_op(int kind, const void* d_items, const int* d_gstart, int nitems, int ngroups,
                RedOut ro, int conv_stage, size_t lds_bytes, hipStream_t s);
 
+// rows per block of the block SteadyGS on grids of mx columns (0: not even one fits the LDS)
+int gsb_block_rows(int mx);
 // the default tile shapes of a product item (rows per work-group of the row stages, columns
 // per work-group of the column stage)
 void conv_default_shape(const ConvItem* c, int* rpg, int* cpg);

@@ -1,0 +1,38 @@
+"""SteadyGS by blocks of rows: interior rows just over 64, 128 and 256 elements (slots of the
+walk's registers), grids that fit 8, 5 and 1 rows per block, last blocks of few rows, and both the
+default and a fixed relaxation.
+
+Tolerance: the same sweeps as the oracle's up to rounding, stopped at eps 1e-9 of the traction's
+rms; with convergence of 0.97 a sweep at worst either is within 32 eps of the solution, so they
+agree to 1e-7 of the largest pressure and the forces to 1e-7 of mu Fn.
+"""
+import numpy as np
+import pytest
+
+from contact_amd import workloads as W
+
+pytestmark = pytest.mark.gpu
+
+CASES = [(9, 11, 0), (69, 17, 0), (69, 10, 3), (134, 12, 0), (262, 11, 0), (450, 6, 0)]
+
+
+@pytest.mark.parametrize("mx,my,gausei", CASES)
+def test_row_widths(cntc, oracle, mx, my, gausei):
+    c = W.base_case(tang=3, norm=1, fn=9e4 * min(1.0, my / mx), cksi=-1e-3, ceta=6e-4, cphi=1e-4, eps=1e-9,
+                    ipotcn=-3, mx=mx, my=my, aa=6.0, bb=6.0 * my / mx, scale=mx / (mx - 4.0), gausei=gausei,
+                    omegah=0.9, omegas=0.95)
+    ire = 942
+    W.apply_case(cntc, ire, 1, c)
+    assert cntc.calculate(ire, 1) == 0
+    p = [a.ravel() for a in cntc.gettractions(ire, 1)]
+    f, its = cntc.getcontactforces(ire, 1), cntc.getiterations(ire, 1)
+    el = cntc.getelementdivision(ire, 1).reshape(my, mx)
+    cntc.finalize(ire)
+    rc, of, P = oracle.solve_case(c)
+    assert rc == 0
+    print(mx, my, "widest row", (el > 0).sum(1).max(), "adhesion", (el == 1).sum(), "iterations", its, P.iters())
+    assert its[4] & 2, "SteadyGS did not run"
+    for a, b in zip(p, P.tractions()):
+        assert np.abs(a - b).max() <= 1e-7 * np.abs(P.tractions()[0]).max()
+    for a, b in zip(f[:3], of[:3]):
+        assert abs(a - b) <= 1e-7 * c["fstat"] * c["fn"]
