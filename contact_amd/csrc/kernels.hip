@@ -17,6 +17,7 @@ namespace cntc {
 
 constexpr int ELEM_THREADS = 256;
 constexpr int ELEM_PER_THREAD = 4;
+constexpr int N_CU = 256;              // compute units
 constexpr int ROW_THREADS = 64;
 constexpr int FFT_THREADS = 256;
 constexpr int MAXK = 12;
@@ -134,7 +135,8 @@ __device__ inline double combine_identity(int mode)
 // wave, lane l taking the partials of groups l, l + 64, ... in order, then a butterfly over the
 // lanes -- an order that depends only on the item's group count, so an item's result is the same
 // whichever other items share the launch.  `extra` receives a copy that later launches read.
-// Must be reached by every thread of the group.
+// Must be reached by every thread of the group; the sums are of the wavefronts w0 .. w0 + nw - 1
+// (default: all).
 //
 // What a reduction adds to a launch is latency.  An item of one group (up to 1024 elements)
 // needs no arrival at all.  With several groups, only the partials pass between groups: they
@@ -146,14 +148,16 @@ __device__ inline double combine_identity(int mode)
 // for 40 x 40.
 template <int K>
 __device__ inline void write_partials(double (&v)[K], int mode, const RedOut& ro, const int* gstart, int it,
-                                      double* extra = nullptr)
+                                      double* extra = nullptr, int w0 = 0, int nw = 0)
 {
     __shared__ double red_lds[16 * MAXK];
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, nwave = (blockDim.x + 63) >> 6;
+    const int lane = threadIdx.x & 63, wave = (threadIdx.x >> 6) - w0, nwave = nw ? nw : (blockDim.x + 63) >> 6;
+    const bool mine = wave >= 0 && wave < nwave;
+    if (mine)
 #pragma unroll
-    for (int k = 0; k < K; k++) v[k] = wave_combine(v[k], mode);
+        for (int k = 0; k < K; k++) v[k] = wave_combine(v[k], mode);
     __syncthreads();
-    if (lane == 0)
+    if (mine && lane == 0)
         for (int k = 0; k < K; k++) red_lds[wave * K + k] = v[k];
     __syncthreads();
     if (wave != 0) return;
@@ -809,7 +813,8 @@ __global__ void __launch_bounds__(ELEM_THREADS) k_st_sa(const StItem* __restrict
 // it loads the recurrence inputs with coalesced reads into LDS, one thread per row runs the
 // recurrence in LDS, and the element-wise rest is done by all threads with coalesced access.
 constexpr int GD_THREADS = 256;
-constexpr int GD_ROW_THREADS = 256;    // threads of update and project
+constexpr int GD_ROW_THREADS = 256;    // threads of project
+constexpr int GD_ELEM_THREADS = ELEM_THREADS * ELEM_PER_THREAD;   // an element per thread
 constexpr int GD_TILE = 2048;          // elements per tile (probe; its sums follow this shape)
 constexpr int GD_TILE_ROW = 1024;      // elements per tile (update, project)
 
@@ -929,7 +934,9 @@ __device__ inline void trcbnd_row(GdCell* lp, const GdBound* lb, int mx)
 
 // The row of a tile that this thread recurs along, from 0; beyond the tile's rows: none.  The
 // lanes of one wave (or its neighbours, for more than 64 rows) do; which wave that is changes
-// with the group, so that the chains of the groups that share a CU run on different SIMDs.
+// with the group, so that the chains of the groups that share a CU run on different SIMDs.  (With
+// the rows divided over four wavefronts, a SIMD each, the chain of a 512 x 512 patch's probe took
+// 128 kcycles instead of 85.)
 __device__ inline int gd_chain_row()
 {
     return (threadIdx.x + blockDim.x - ((blockIdx.x >> 8) & 3) * 64) % blockDim.x;
@@ -1114,8 +1121,15 @@ __global__ void __launch_bounds__(GD_ROW_THREADS, 4) k_gd_project(const GdItem* 
 // dp + alpha dv, then the residual terms of the new orientation.  Returns
 // (rho, c0adh, c1adh, c0slp, c1slp, c2slp) and, when I.first, also
 // (sum r^2, sum r.q dscl, sum_int (dscl q)^2, sum_int r^2).
-__global__ void __launch_bounds__(GD_THREADS) k_gd_probe(const GdItem* __restrict__ items, const int* __restrict__ gstart,
-                                                         int nitems, RedOut ro)
+//
+// Latency-bound: the row chain, then atan2, cos and sin per element.  The terms take all T
+// threads; each element's are left in its LDS cells and added up by 256 of the threads, element
+// t, t + 256, ... each, so that the sums do not depend on T.  With 256 threads for
+// all of it, eight elements in turn each: 26.4 us a launch for a mix of sides 20 to 256, 25.2 us
+// so; 512 x 512 88.9 and 88.2 us (HIP events, about 4 us of each their own).
+template <int T>
+__global__ void __launch_bounds__(T, 4) k_gd_probe(const GdItem* __restrict__ items, const int* __restrict__ gstart,
+                                                   int nitems, RedOut ro)
 {
     extern __shared__ double gd_lds[];
     int it = find_item(gstart, nitems, blockIdx.x);
@@ -1124,18 +1138,18 @@ __global__ void __launch_bounds__(GD_THREADS) k_gd_probe(const GdItem* __restric
     const int R = gd_rows_per_tile(mx, I.my, GD_TILE);
     const int row0 = (blockIdx.x - gstart[it]) * R;
     const int nrow = min(R, I.my - row0);
-    const int ne = nrow * mx;
+    const int ne = nrow * mx;        // at most GD_TILE (grids have at most 2048 columns)
     const size_t g0 = (size_t)row0 * mx;
     const double a = I.alpha;
-    GdCell* lp = (GdCell*)gd_lds;    // dp + alpha dv, then the new p
+    GdCell* lp = (GdCell*)gd_lds;    // dp + alpha dv, then the new p, then the terms
     GdBound* lb = (GdBound*)(lp + R * S);
-    constexpr int U = 4;
-    for (int e0 = threadIdx.x; e0 < ne; e0 += U * GD_THREADS) {
+    constexpr int U = GD_TILE / T;
+    {
         int8_t st[U];
         double pn[U], dx[U], dy[U], vx[U], vy[U];
 #pragma unroll
         for (int u = 0; u < U; u++) {
-            const int e = e0 + u * GD_THREADS;
+            const int e = threadIdx.x + u * T;
             const size_t i = g0 + (e < ne ? e : 0);
             st[u] = as_global(I.el)[i];
             pn[u] = as_global(I.pn)[i];
@@ -1146,7 +1160,7 @@ __global__ void __launch_bounds__(GD_THREADS) k_gd_probe(const GdItem* __restric
         }
 #pragma unroll
         for (int u = 0; u < U; u++) {
-            const int e = e0 + u * GD_THREADS;
+            const int e = threadIdx.x + u * T;
             const int r = e / mx, l = r * S + (e - r * mx);
             const GdCell c{fma(a, vx[u], dx[u]), fma(a, vy[u], dy[u])};
             const GdBound b = gd_bound(I.mu * pn[u], st[u]);
@@ -1159,19 +1173,15 @@ __global__ void __launch_bounds__(GD_THREADS) k_gd_probe(const GdItem* __restric
     // the element terms' inputs: the first element's are on their way during the row recurrence,
     // then each element's during the arithmetic of the one before
     struct Terms {
-        double dscl, sx, sy, qx, qy, rx, ry, nx, ny, vx, vy;
+        double sx, sy, qx, qy, nx, ny, vx, vy;
     };
-    const int first = I.first;
     auto fetch = [&](int e) {
         const size_t ii = g0 + (e < ne ? e : 0);
         Terms t;
-        t.dscl = as_global(I.dscl)[ii];
         t.sx = as_global(I.sx)[ii];
         t.sy = as_global(I.sy)[ii];
         t.qx = as_global(I.qx)[ii];
         t.qy = as_global(I.qy)[ii];
-        t.rx = first ? as_global(I.rx)[ii] : 0.0;
-        t.ry = first ? as_global(I.ry)[ii] : 0.0;
         t.nx = as_global(I.nx)[ii];
         t.ny = as_global(I.ny)[ii];
         t.vx = as_global(I.vx)[ii];
@@ -1184,62 +1194,111 @@ __global__ void __launch_bounds__(GD_THREADS) k_gd_probe(const GdItem* __restric
         const int l0 = row * S;
         trcbnd_row(lp + l0, lb + l0, mx);
     }
+    // the last 256 threads sum, and do the sums that need no chain meanwhile
+    constexpr int T0 = T - GD_THREADS, V = GD_TILE / GD_THREADS;
+    const int t0 = (int)threadIdx.x - T0;
+    __shared__ double early[4][GD_THREADS];   // (not held in registers over the terms)
+    if (I.first && t0 >= 0) {
+        double acc[4] = {0.0, 0.0, 0.0, 0.0};
+#pragma unroll 4
+        for (int e = t0; e < ne; e += GD_THREADS) {
+            const size_t ii = g0 + e;
+            const double rx = as_global(I.rx)[ii], ry = as_global(I.ry)[ii];
+            const double qx = as_global(I.qx)[ii], qy = as_global(I.qy)[ii];
+            const double dscl = as_global(I.dscl)[ii];
+            acc[0] += rx * rx + ry * ry;
+            acc[1] += (rx * qx + ry * qy) * dscl;
+            if (as_global(I.el)[ii] >= ADHES) {
+                acc[2] += dscl * dscl * (qx * qx + qy * qy);
+                acc[3] += rx * rx + ry * ry;
+            }
+        }
+#pragma unroll
+        for (int k = 0; k < 4; k++) early[k][t0] = acc[k];
+    }
     __syncthreads();
-    double acc[10] = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
     const double tiny = 1e-12;
-    for (int e = threadIdx.x; e < ne; e += GD_THREADS) {
+    for (int e = threadIdx.x; e < ne; e += T) {
         int r = e / mx, l = r * S + (e - r * mx);
         const GdBound b = lb[l];
         const int8_t st = gd_state(b);
         const Terms t = ahead;
-        if (e + GD_THREADS < ne) ahead = fetch(e + GD_THREADS);
-        double dscl = t.dscl;
-        double sx = t.sx, sy = t.sy, qx = t.qx, qy = t.qy;
-        if (first) {
-            double rx = t.rx, ry = t.ry;
-            acc[6] += rx * rx + ry * ry;
-            acc[7] += (rx * qx + ry * qy) * dscl;
-            if (st >= ADHES) {
-                acc[8] += dscl * dscl * (qx * qx + qy * qy);
-                acc[9] += rx * rx + ry * ry;
+        if (e + T < ne) ahead = fetch(e + T);
+        // the terms: in adhesion e^2 >= 0 and two factors of 2 dscl^2; in slip -|e| (sign bit
+        // set) and three
+        GdCell c{0.0, 0.0};
+        GdBound d{0.0, 0.0};
+        if (st == ADHES || st == SLIP) {
+            double sx = t.sx, sy = t.sy, qx = t.qx, qy = t.qy;
+            double px = lp[l].x, py = lp[l].y, g = fabs(b.c);
+            double txo = -t.ny, tyo = t.nx;
+            double vt = t.vx * txo + t.vy * tyo;
+            double dth_da = (g * vt) / (fmax(tiny, g * g) + a * a * vt * vt);
+            double nxn, nyn;
+            nt_from_p(px, py, nxn, nyn);
+            double txn = -nyn, tyn = nxn;
+            double sn = sx * nxn + sy * nyn;
+            int8_t elnew = st;
+            if (elnew == SLIP && sn > 0.0) elnew = ADHES;
+            double stt = sx * txn + sy * tyn, rt = -stt;
+            double qn = qx * nxn + qy * nyn, qt = qx * txn + qy * tyn;
+            if (elnew == ADHES) {
+                double ex = sx + a * qx, ey = sy + a * qy;
+                c.x = ex * ex + ey * ey;
+                c.y = sx * qx + sy * qy;
+                d.c = qx * qx + qy * qy;
+            } else {
+                double ex = stt + a * qt;
+                c.x = copysign(ex, -1.0);
+                c.y = rt * qt - rt * sn * dth_da;
+                d.c = -qt * qt + qt * sn * dth_da - rt * qn * dth_da;
+                d.lim = qt * qn * dth_da;
             }
         }
-        if (st != ADHES && st != SLIP) continue;
-        double px = lp[l].x, py = lp[l].y, g = fabs(b.c);
-        double txo = -t.ny, tyo = t.nx;
-        double vt = t.vx * txo + t.vy * tyo;
-        double dth_da = (g * vt) / (fmax(tiny, g * g) + a * a * vt * vt);
-        double nxn, nyn;
-        nt_from_p(px, py, nxn, nyn);
-        double txn = -nyn, tyn = nxn;
-        double sn = sx * nxn + sy * nyn;
-        int8_t elnew = st;
-        if (elnew == SLIP && sn > 0.0) elnew = ADHES;
-        double stt = sx * txn + sy * tyn, rt = -stt;
-        double qn = qx * nxn + qy * nyn, qt = qx * txn + qy * tyn;
-        double d2 = dscl * dscl;
-        if (elnew == ADHES) {
-            acc[1] += 2.0 * d2 * (sx * qx + sy * qy);
-            acc[2] += 2.0 * d2 * (qx * qx + qy * qy);
-            double ex = sx + a * qx, ey = sy + a * qy;
-            acc[0] += d2 * (ex * ex + ey * ey);
-        } else {
-            acc[3] -= 2.0 * d2 * (rt * qt - rt * sn * dth_da);
-            acc[4] -= 2.0 * d2 * (-qt * qt + qt * sn * dth_da - rt * qn * dth_da);
-            acc[5] -= 2.0 * d2 * (qt * qn * dth_da);
-            double ex = stt + a * qt;
-            acc[0] += d2 * ex * ex;
-        }
+        lp[l] = c;
+        lb[l] = d;
     }
-    write_partials<10>(acc, 0, ro, gstart, it);
+    double acc[10] = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
+    double dscl[V];
+    if (t0 >= 0)
+#pragma unroll
+        for (int v = 0; v < V; v++) {
+            const int e = t0 + v * GD_THREADS;
+            dscl[v] = as_global(I.dscl)[g0 + (e < ne ? e : 0)];
+        }
+    __syncthreads();
+    if (I.first && t0 >= 0)
+#pragma unroll
+        for (int k = 0; k < 4; k++) acc[6 + k] = early[k][t0];
+    if (t0 >= 0)
+#pragma unroll
+        for (int v = 0; v < V; v++) {
+            const int e = t0 + v * GD_THREADS;
+            if (e >= ne) break;
+            const int r = e / mx, l = r * S + (e - r * mx);
+            const GdCell c = lp[l];
+            const GdBound d = lb[l];
+            const bool slip = signbit(c.x);
+            const double d2 = dscl[v] * dscl[v], dd = 2.0 * d2;
+            acc[0] = fma(slip ? d2 * c.x : d2, c.x, acc[0]);
+            const double a1 = fma(dd, c.y, acc[1]), a2 = fma(dd, d.c, acc[2]);
+            const double a3 = fma(-dd, c.y, acc[3]), a4 = fma(-dd, d.c, acc[4]), a5 = fma(-dd, d.lim, acc[5]);
+            acc[1] = slip ? acc[1] : a1;
+            acc[2] = slip ? acc[2] : a2;
+            acc[3] = slip ? a3 : acc[3];
+            acc[4] = slip ? a4 : acc[4];
+            acc[5] = slip ? a5 : acc[5];
+        }
+    write_partials<10>(acc, 0, ro, gstart, it, nullptr, T0 / 64, GD_THREADS / 64);
 }
 
 // pold = p; dp += alpha dv on the interior; apply_trcbnd (src/gdsteady.f90:807-847); n from p.
 // No sums, so tiles and threads are free of the probe's: half its tile, so that every CU has one
 // at 512 x 512: 118 us a launch with the plain row loop in the probe's tile, 73 us so; 1024 x
 // 1024: 171 and 162 us; 40 x 40: 22 and 16 us.
-__global__ void __launch_bounds__(GD_ROW_THREADS, 4) k_gd_update(const GdItem* __restrict__ items, const int* __restrict__ gstart,
-                                                              int nitems, RedOut ro)
+template <int T>
+__global__ void __launch_bounds__(T, 4) k_gd_update(const GdItem* __restrict__ items, const int* __restrict__ gstart,
+                                                    int nitems, RedOut ro)
 {
     extern __shared__ double gd_lds[];
     int it = find_item(gstart, nitems, blockIdx.x);
@@ -1252,13 +1311,13 @@ __global__ void __launch_bounds__(GD_ROW_THREADS, 4) k_gd_update(const GdItem* _
     const size_t g0 = (size_t)row0 * mx;
     GdCell* lp = (GdCell*)gd_lds;    // dp + alpha dv, then the new p
     GdBound* lb = (GdBound*)(lp + R * S);
-    constexpr int U = 2;
-    for (int e0 = threadIdx.x; e0 < ne; e0 += U * GD_ROW_THREADS) {
+    constexpr int U = T <= 512 ? 2 : 1;
+    for (int e0 = threadIdx.x; e0 < ne; e0 += U * T) {
         int8_t st[U];
         double pn[U], dx[U], dy[U], vx[U], vy[U], px[U], py[U];
 #pragma unroll
         for (int u = 0; u < U; u++) {
-            const int e = e0 + u * GD_ROW_THREADS;
+            const int e = e0 + u * T;
             const size_t i = g0 + (e < ne ? e : 0);
             st[u] = as_global(I.el)[i];
             pn[u] = as_global(I.pn)[i];
@@ -1271,7 +1330,7 @@ __global__ void __launch_bounds__(GD_ROW_THREADS, 4) k_gd_update(const GdItem* _
         }
 #pragma unroll
         for (int u = 0; u < U; u++) {
-            const int e = e0 + u * GD_ROW_THREADS;
+            const int e = e0 + u * T;
             if (e >= ne) break;
             const int r = e / mx, ix = e - r * mx, l = r * S + ix;
             const size_t i = g0 + e;
@@ -1294,7 +1353,7 @@ __global__ void __launch_bounds__(GD_ROW_THREADS, 4) k_gd_update(const GdItem* _
         trcbnd_row(lp + l0, lb + l0, mx);
     }
     __syncthreads();
-    for (int e = threadIdx.x; e < ne; e += GD_ROW_THREADS) {
+    for (int e = threadIdx.x; e < ne; e += T) {
         const int r = e / mx, ix = e - r * mx, l = r * S + ix;
         const size_t ii = g0 + e;
         const GdCell p = lp[l];
@@ -1485,49 +1544,54 @@ __device__ void elmtrc(int8_t& el, const double c11, const double c12, const dou
     s[1] = siy;
 }
 
-// element-state moves after a GD step (src/gdsteady.f90:375-418); returns #changes
-__global__ void __launch_bounds__(ELEM_THREADS) k_gd_moves(const GdItem* __restrict__ items, const int* __restrict__ gstart,
-                                                           int nitems, RedOut ro)
+// element-state moves after a GD step (src/gdsteady.f90:375-418); returns #changes.  An element
+// per thread: latency-bound by the slip elements' 2x2 problem.  Only the signs and states that
+// follow from its solution are used, so it is solved on the latency path (elmtrc, scale_dir).
+// With four elements in turn and the general problem 20.3 us a launch for a mix of sides 20 to 256,
+// 10.1 us so; 1024 x 1024 33.2 and 26.5 us (HIP events, about 4 us of each their own).
+__global__ void __launch_bounds__(GD_ELEM_THREADS) k_gd_moves(const GdItem* __restrict__ items, const int* __restrict__ gstart,
+                                                              int nitems, RedOut ro)
 {
     int it = find_item(gstart, nitems, blockIdx.x);
     const GdItem& I = items[it];
-    int base = (blockIdx.x - gstart[it]) * ELEM_THREADS * ELEM_PER_THREAD;
+    const int i = (blockIdx.x - gstart[it]) * GD_ELEM_THREADS + threadIdx.x;
     double acc[1] = {0.0};
     const double tiny = 1e-12;
-    for (int e = 0; e < ELEM_PER_THREAD; e++) {
-        int i = base + e * ELEM_THREADS + threadIdx.x;
-        if (i >= I.n) break;
-        int8_t s = I.el[i];
-        double g = I.mu * I.pn[i];
+    const size_t ii = i < I.n ? i : 0;
+    const int8_t s = as_global(I.el)[ii];
+    double pr[3] = {as_global(I.px)[ii], as_global(I.py)[ii], as_global(I.pn)[ii]};
+    double si[2] = {as_global(I.sx)[ii], as_global(I.sy)[ii]};
+    const double nx = as_global(I.nx)[ii], ny = as_global(I.ny)[ii], dscl = as_global(I.dscl)[ii];
+    if (i < I.n) {
+        const double g = I.mu * pr[2];
         if (s == ADHES) {
-            double ptabs = sqrt(I.px[i] * I.px[i] + I.py[i] * I.py[i]);
+            double ptabs = sqrt(pr[0] * pr[0] + pr[1] * pr[1]);
             if (ptabs >= g - tiny) {
-                I.el[i] = SLIP;
-                acc[0] += 1.0;
+                as_global(I.el)[ii] = SLIP;
+                acc[0] = 1.0;
             }
         } else if (s == SLIP) {
-            double pr[3] = {I.px[i], I.py[i], I.pn[i]};
-            double si[2] = {I.sx[i], I.sy[i]};
+            const double snrm = nx * si[0] + ny * si[1];
             int8_t elopt = s;
-            elmtrc(elopt, I.c11, I.c12, I.c21, I.c22, 1e-6, pr, I.mu, si);
-            double snrm = I.nx[i] * I.sx[i] + I.ny[i] * I.sy[i];
-            double cosdth = (I.nx[i] * pr[0] + I.ny[i] * pr[1]) / g;
-            if ((snrm > 0.0 && (I.dscl[i] >= 0.001 || elopt == ADHES)) || cosdth <= -0.5) {
-                I.el[i] = ADHES;
-                acc[0] += 1.0;
+            elmtrc(elopt, I.c11, I.c12, I.c21, I.c22, 1e-6, pr, I.mu, si, 1.0, 1.0, true);
+            double cosdth = (nx * pr[0] + ny * pr[1]) / g;
+            if ((snrm > 0.0 && (dscl >= 0.001 || elopt == ADHES)) || cosdth <= -0.5) {
+                as_global(I.el)[ii] = ADHES;
+                acc[0] = 1.0;
             }
         }
     }
-    write_partials<1>(acc, 0, ro, gstart, it);
+    write_partials<1>(acc, 0, ro, gstart, it);   // (whole numbers: exact in any order)
 }
 
 // angle-split of a slip element (compute_diagscaling, src/gdsteady.f90:927-980); returns
 // false when the angle error stays below tiny_err (elnew/fac_s then keep earlier values)
-__device__ inline bool gd_slip_split(const GdItem& I, int ii, int8_t& elnew, double& fac_s)
+__device__ inline bool gd_slip_split(const GdItem& I, const double px, const double py, const double pn,
+                                     const double sx, const double sy, int8_t& elnew, double& fac_s)
 {
     const double tiny_err = 1e-6, PI = 3.14159265358979323846;
-    double pr[3] = {I.px[ii], I.py[ii], I.pn[ii]};
-    double si[2] = {I.sx[ii], I.sy[ii]};
+    double pr[3] = {px, py, pn};
+    double si[2] = {sx, sy};
     double th_p0 = atan2(pr[1], pr[0]);
     double th_s0 = atan2(-si[1], -si[0]);
     double err_0 = th_s0 - th_p0;
@@ -1535,8 +1599,8 @@ __device__ inline bool gd_slip_split(const GdItem& I, int ii, int8_t& elnew, dou
     if (fabs(err_0) <= tiny_err) {
         pr[0] = I.mu * pr[2] * cos(th_p0 + 0.1);
         pr[1] = I.mu * pr[2] * sin(th_p0 + 0.1);
-        si[0] = I.sx[ii] + I.c11 * (pr[0] - I.px[ii]) + I.c12 * (pr[1] - I.py[ii]);
-        si[1] = I.sy[ii] + I.c21 * (pr[0] - I.px[ii]) + I.c22 * (pr[1] - I.py[ii]);
+        si[0] = sx + I.c11 * (pr[0] - px) + I.c12 * (pr[1] - py);
+        si[1] = sy + I.c21 * (pr[0] - px) + I.c22 * (pr[1] - py);
         th_p0 = atan2(pr[1], pr[0]);
         th_s0 = atan2(-si[1], -si[0]);
         err_0 = th_s0 - th_p0;
@@ -1557,72 +1621,107 @@ __device__ inline bool gd_slip_split(const GdItem& I, int ii, int8_t& elnew, dou
 
 // compute_diagscaling and the scaled residual (src/gdsteady.f90:901-1042, 429-439); when
 // not I.first also pold -= p on the interior.  Returns (sum (pold)^2, sum p^2, sum_int r^2).
-__global__ void __launch_bounds__(ELEM_THREADS) k_gd_diagres(const GdItem* __restrict__ items, const int* __restrict__ gstart,
-                                                             int nitems, RedOut ro)
+// An element per thread: latency-bound by the slip elements' angles and 2x2 problem.  The start
+// of an element's run of adhesion is found from the states of the wavefront, 64 at a time.  The
+// sums are those of 256 threads with elements t, t + 256, ... each.  With four elements in turn and the run walked element by element 43.4 us a launch for a
+// mix of sides 20 to 256, 20.2 us so; 40 x 40 29.6 and 18.6, 1024 x 1024 65.7 and 73.5 us (HIP
+// events, about 4 us of each their own).
+__global__ void __launch_bounds__(GD_ELEM_THREADS) k_gd_diagres(const GdItem* __restrict__ items, const int* __restrict__ gstart,
+                                                                int nitems, RedOut ro)
 {
+    __shared__ double con[3][GD_ELEM_THREADS];
     int it = find_item(gstart, nitems, blockIdx.x);
     const GdItem& I = items[it];
-    int base = (blockIdx.x - gstart[it]) * ELEM_THREADS * ELEM_PER_THREAD;
-    double acc[3] = {0.0, 0.0, 0.0};
-    for (int e = 0; e < ELEM_PER_THREAD; e++) {
-        int i = base + e * ELEM_THREADS + threadIdx.x;
-        if (i >= I.n) break;
-        int8_t s = I.el[i];
+    const int mx = I.mx, i = (blockIdx.x - gstart[it]) * GD_ELEM_THREADS + threadIdx.x;
+    const bool in = i < I.n;
+    const size_t ii = in ? i : 0;
+    const int8_t s = in ? as_global(I.el)[ii] : EXTER;
+    const double px = as_global(I.px)[ii], py = as_global(I.py)[ii], pn = as_global(I.pn)[ii];
+    const double sx = as_global(I.sx)[ii], sy = as_global(I.sy)[ii];
+    const double nx = as_global(I.nx)[ii], ny = as_global(I.ny)[ii];
+    double ox = 0.0, oy = 0.0;
+    if (!I.first) {
+        ox = as_global(I.poldx)[ii];
+        oy = as_global(I.poldy)[ii];
+    }
+    double dscl = as_global(I.dscl)[ii];
+    // the run of adhesion that this element ends: its first element is the nearest one, at or
+    // before this one, that begins the row or follows an element not in adhesion
+    auto begins = [&](int j) { return j % mx == 0 || as_global(I.el)[j - 1] != ADHES; };
+    const int lane = threadIdx.x & 63, w0 = i - lane;
+    const unsigned long long stop = __builtin_amdgcn_ballot_w64(!in || begins(i));
+    const unsigned long long mine = stop & (~0ull >> (63 - lane));
+    int start = w0 + 63 - __clzll((long long)mine);
+    if (!(stop & 1)) {
+        int prev = 0;
+        for (int c = w0 - 64; c >= 0; c -= 64) {
+            const unsigned long long b = __builtin_amdgcn_ballot_w64(begins(c + lane));
+            if (b) {
+                prev = c + 63 - __clzll((long long)b);
+                break;
+            }
+        }
+        if (!mine) start = prev;
+    }
+    double rx = 0.0, ry = 0.0, c0 = 0.0, c1 = 0.0, c2 = 0.0;
+    if (in) {
         int8_t elnew = EXTER;
         double fac_s = 0.0;
         bool have = false;
-        if (s == SLIP) have = gd_slip_split(I, i, elnew, fac_s);
+        if (s == SLIP) have = gd_slip_split(I, px, py, pn, sx, sy, elnew, fac_s);
         if (s == SLIP && !have) {
             // the reference keeps elnew/fac_s of the last slip element it split
             for (int j = i - 1; j >= 0; j--) {
                 if (I.el[j] != SLIP) continue;
-                if (gd_slip_split(I, j, elnew, fac_s)) break;
+                if (gd_slip_split(I, I.px[j], I.py[j], I.pn[j], I.sx[j], I.sy[j], elnew, fac_s)) break;
             }
         }
-        double dscl = I.dscl[i];
         if (s == SLIP && elnew == SLIP) {
             dscl = I.d_slp * pow(fac_s, I.pow_s);
         } else if (s == ADHES || (s == SLIP && elnew == ADHES)) {
-            int ix = i % I.mx + 1;
-            int jx = ix;
-            while (jx > 1 && I.el[i - ix + jx - 1] == ADHES) jx--;
+            const int run = i - start;
             double dnew;
             if (I.d_cns < I.d_ifc)
-                dnew = fmax(I.d_cns, I.d_ifc + (ix - jx - 1) * fmin(0.0, I.d_lin));
+                dnew = fmax(I.d_cns, I.d_ifc + (run - 1) * fmin(0.0, I.d_lin));
             else
-                dnew = fmin(I.d_cns, I.d_ifc + (ix - jx - 1) * fmax(0.0, I.d_lin));
+                dnew = fmin(I.d_cns, I.d_ifc + (run - 1) * fmax(0.0, I.d_lin));
             dscl = fmin(50.0 * dscl, dnew);
         } else if (s != ADHES) {
             dscl = 0.0;
         }
-        I.dscl[i] = dscl;
-        double rx = 0.0, ry = 0.0;
+        as_global(I.dscl)[ii] = dscl;
         if (s == ADHES) {
-            rx = -I.sx[i] * dscl;
-            ry = -I.sy[i] * dscl;
+            rx = -sx * dscl;
+            ry = -sy * dscl;
         } else if (s == SLIP) {
-            double tx = -I.ny[i], ty = I.nx[i];
-            double st = tx * I.sx[i] + ty * I.sy[i];
+            double tx = -ny, ty = nx;
+            double st = tx * sx + ty * sy;
             rx = -st * tx * dscl;
             ry = -st * ty * dscl;
         }
-        I.rx[i] = rx;
-        I.ry[i] = ry;
-        double px = I.px[i], py = I.py[i];
+        as_global(I.rx)[ii] = rx;
+        as_global(I.ry)[ii] = ry;
         if (!I.first) {
-            double ox = I.poldx[i], oy = I.poldy[i];
             if (s >= ADHES) {
                 ox -= px;
                 oy -= py;
-                I.poldx[i] = ox;
-                I.poldy[i] = oy;
+                as_global(I.poldx)[ii] = ox;
+                as_global(I.poldy)[ii] = oy;
             }
-            acc[0] += ox * ox + oy * oy;
+            c0 = ox * ox + oy * oy;
         }
-        acc[1] += px * px + py * py;
-        if (s >= ADHES) acc[2] += rx * rx + ry * ry;
+        c1 = px * px + py * py;
+        if (s >= ADHES) c2 = rx * rx + ry * ry;
     }
-    write_partials<3>(acc, 0, ro, gstart, it);
+    con[0][threadIdx.x] = c0;
+    con[1][threadIdx.x] = c1;
+    con[2][threadIdx.x] = c2;
+    __syncthreads();
+    double acc[3] = {0.0, 0.0, 0.0};
+    if (threadIdx.x < ELEM_THREADS)
+        for (int k = 0; k < 3; k++)
+            for (int e = 0; e < ELEM_PER_THREAD; e++) acc[k] += con[k][e * ELEM_THREADS + threadIdx.x];
+    write_partials<3>(acc, 0, ro, gstart, it, nullptr, 0, ELEM_THREADS / 64);
 }
 
 // ------------------------------------------------------------------------------------------
@@ -4402,10 +4501,17 @@ void launch_op(int kind, const void* d_items, const int* d_gstart, int nitems, i
     case OP_GSB_WALK: hipLaunchKernelGGL(k_gsb_walk, ge, dim3(GSB_THREADS), lds_bytes, s, (const GsbItem*)d_items, d_gstart, nitems, ro); break;
     case OP_GSB_CHECK: hipLaunchKernelGGL(k_gsb_check, ge, dim3(GSB_THREADS), 0, s, (const GsbItem*)d_items, d_gstart, nitems, ro); break;
     case OP_GD_PROJECT: hipLaunchKernelGGL(k_gd_project, ge, dim3(GD_ROW_THREADS), lds_bytes, s, (const GdItem*)d_items, d_gstart, nitems, ro); break;
-    case OP_GD_PROBE: hipLaunchKernelGGL(k_gd_probe, ge, dim3(GD_THREADS), lds_bytes, s, (const GdItem*)d_items, d_gstart, nitems, ro); break;
-    case OP_GD_UPDATE: hipLaunchKernelGGL(k_gd_update, ge, dim3(GD_ROW_THREADS), lds_bytes, s, (const GdItem*)d_items, d_gstart, nitems, ro); break;
-    case OP_GD_MOVES: hipLaunchKernelGGL(k_gd_moves, ge, te, 0, s, (const GdItem*)d_items, d_gstart, nitems, ro); break;
-    case OP_GD_DIAGRES: hipLaunchKernelGGL(k_gd_diagres, ge, te, 0, s, (const GdItem*)d_items, d_gstart, nitems, ro); break;
+    // with a CU to each group the most threads it can have; else those of which two groups share one
+    case OP_GD_PROBE:
+        if (ngroups <= N_CU) hipLaunchKernelGGL(k_gd_probe<1024>, ge, dim3(1024), lds_bytes, s, (const GdItem*)d_items, d_gstart, nitems, ro);
+        else hipLaunchKernelGGL(k_gd_probe<512>, ge, dim3(512), lds_bytes, s, (const GdItem*)d_items, d_gstart, nitems, ro);
+        break;
+    case OP_GD_UPDATE:
+        if (ngroups <= N_CU) hipLaunchKernelGGL(k_gd_update<1024>, ge, dim3(1024), lds_bytes, s, (const GdItem*)d_items, d_gstart, nitems, ro);
+        else hipLaunchKernelGGL(k_gd_update<256>, ge, dim3(256), lds_bytes, s, (const GdItem*)d_items, d_gstart, nitems, ro);
+        break;
+    case OP_GD_MOVES: hipLaunchKernelGGL(k_gd_moves, ge, dim3(GD_ELEM_THREADS), 0, s, (const GdItem*)d_items, d_gstart, nitems, ro); break;
+    case OP_GD_DIAGRES: hipLaunchKernelGGL(k_gd_diagres, ge, dim3(GD_ELEM_THREADS), 0, s, (const GdItem*)d_items, d_gstart, nitems, ro); break;
     case OP_SETUP: hipLaunchKernelGGL(k_setup, ge, te, 0, s, (const SetupItem*)d_items, d_gstart, nitems, ro); break;
     case OP_FORCES: hipLaunchKernelGGL(k_forces, ge, te, 0, s, (const SetupItem*)d_items, d_gstart, nitems, ro); break;
     case OP_STDYGS:
