@@ -19,6 +19,7 @@ constexpr int ELEM_THREADS = 256;
 constexpr int ELEM_PER_THREAD = 4;
 constexpr int N_CU = 256;              // compute units
 constexpr int ROW_THREADS = 64;
+constexpr int AIJ_THREADS = 1024;
 constexpr int FFT_THREADS = 256;
 constexpr int MAXK = 12;
 
@@ -488,34 +489,55 @@ __global__ void __launch_bounds__(ELEM_THREADS) k_sn_final(const NcgItem* __rest
 
 // gf3_AijPj with unit tractions at one element: sum over rows jy of the coefficients for
 // jx in [row1st-1, rowlst+1] of the current contact area (src/m_aijpj.f90:158-185,
-// src/m_gridfunc.f90:582-637).  One group per item, one thread per row.
-__global__ void __launch_bounds__(ROW_THREADS) k_aij_ones(const AijItem* __restrict__ items, const int* __restrict__ gstart,
+// src/m_gridfunc.f90:582-637).  A group per 64 rows.
+//
+// Latency-bound: each wavefront finds the ranges of four rows from 64 states at a time, then the
+// lanes of the first add up a row each, in order, sixteen coefficients on their way together.
+// With the states and coefficients of a row read one after the other 565 us for
+// 1024 x 1024, 75 us so; 18 and 6.5 us for 40 x 40 (HIP events, about 4 us of each their own).
+__global__ void __launch_bounds__(AIJ_THREADS) k_aij_ones(const AijItem* __restrict__ items, const int* __restrict__ gstart,
                                                           int nitems, RedOut ro)
 {
+    __shared__ int range[ROW_THREADS][2];
     int it = find_item(gstart, nitems, blockIdx.x);
     const AijItem& I = items[it];
-    double acc[1] = {0.0};
-    int rows_per_group = ROW_THREADS;
-    int jy0 = (blockIdx.x - gstart[it]) * rows_per_group;
-    int jy = jy0 + threadIdx.x + 1;   // 1-based row
-    if (jy <= I.my) {
-        const int8_t* row = I.el + (size_t)(jy - 1) * I.mx;
-        int first = 1;
-        while (row[first - 1] <= EXTER && first != I.mx) first++;
-        int last = 0;
-        for (int ix = first; ix <= I.mx; ix++)
-            if (row[ix - 1] >= ADHES) last = ix;
-        int j0 = first - 1 < 1 ? 1 : first - 1;
-        int j1 = last + 1 > I.mx ? I.mx : last + 1;
-        double rowsum = 0.0;
-        for (int jx = j0; jx <= j1; jx++) {
-            int dx = I.ix - jx, dy = I.iy - jy;
-            if (dx < -I.cf_mx || dx >= I.cf_mx || dy < -I.cf_my || dy >= I.cf_my) continue;
-            rowsum += I.cf[(size_t)(dy + I.cf_my) * (2 * I.cf_mx) + (dx + I.cf_mx)];
+    const int mx = I.mx, jy0 = (blockIdx.x - gstart[it]) * ROW_THREADS, lane = threadIdx.x & 63;
+    for (int r = threadIdx.x >> 6; r < ROW_THREADS && jy0 + r < I.my; r += AIJ_THREADS / 64) {
+        const auto row = as_global(I.el) + (size_t)(jy0 + r) * mx;
+        int first = mx, last = 0;   // (1-based)
+        for (int c = 0; c < mx; c += 64) {
+            const int8_t e = c + lane < mx ? row[c + lane] : EXTER;
+            const unsigned long long any = __builtin_amdgcn_ballot_w64(e > EXTER);
+            const unsigned long long con = __builtin_amdgcn_ballot_w64(e >= ADHES);
+            if (any) first = min(first, c + __ffsll((long long)any));
+            if (con) last = c + 64 - __clzll((long long)con);
         }
-        acc[0] = rowsum;
+        if (lane == 0) {
+            range[r][0] = max(1, first - 1);
+            range[r][1] = min(mx, last + 1);
+        }
     }
-    write_partials<1>(acc, 0, ro, gstart, it);
+    __syncthreads();
+    double acc[1] = {0.0};
+    const int jy = jy0 + threadIdx.x + 1;   // 1-based row
+    if (threadIdx.x < ROW_THREADS && jy <= I.my) {
+        const int dy = I.iy - jy;
+        const int j0 = max(range[threadIdx.x][0], I.ix - I.cf_mx + 1), j1 = min(range[threadIdx.x][1], I.ix + I.cf_mx);
+        if (dy >= -I.cf_my && dy < I.cf_my) {
+            const auto cf = as_global(I.cf) + (size_t)(dy + I.cf_my) * (2 * I.cf_mx) + (I.ix + I.cf_mx);
+            constexpr int U = 16;
+            double rowsum = 0.0;
+            for (int jx = j0; jx <= j1; jx += U) {
+                double v[U];
+#pragma unroll
+                for (int u = 0; u < U; u++) v[u] = cf[-min(jx + u, j1)];
+#pragma unroll
+                for (int u = 0; u < U; u++) rowsum = jx + u <= j1 ? rowsum + v[u] : rowsum;
+            }
+            acc[0] = rowsum;
+        }
+    }
+    write_partials<1>(acc, 0, ro, gstart, it, nullptr, 0, 1);
 }
 
 // ------------------------------------------------------------------------------------------
@@ -4516,7 +4538,7 @@ void launch_op(int kind, const void* d_items, const int* d_gstart, int nitems, i
                RedOut ro, int conv_stage, size_t lds_bytes, hipStream_t s)
 {
     if (ngroups <= 0) return;
-    dim3 ge(ngroups), te(ELEM_THREADS), tr(ROW_THREADS), tf(FFT_THREADS);
+    dim3 ge(ngroups), te(ELEM_THREADS), tf(FFT_THREADS);
     switch (kind) {
     case OP_VEC: hipLaunchKernelGGL(k_vec, ge, te, 0, s, (const VecItem*)d_items, d_gstart, nitems, ro); break;
     case OP_NCG_NEGPN: hipLaunchKernelGGL(k_ncg_negpn, ge, te, 0, s, (const NcgItem*)d_items, d_gstart, nitems, ro); break;
@@ -4526,7 +4548,7 @@ void launch_op(int kind, const void* d_items, const int* d_gstart, int nitems, i
     case OP_SN_CONTRACT: hipLaunchKernelGGL(k_sn_contract, ge, te, 0, s, (const NcgItem*)d_items, d_gstart, nitems, ro); break;
     case OP_SN_EXPAND: hipLaunchKernelGGL(k_sn_expand, ge, te, 0, s, (const NcgItem*)d_items, d_gstart, nitems, ro); break;
     case OP_SN_FINAL: hipLaunchKernelGGL(k_sn_final, ge, te, 0, s, (const NcgItem*)d_items, d_gstart, nitems, ro); break;
-    case OP_AIJ_ONES: hipLaunchKernelGGL(k_aij_ones, ge, tr, 0, s, (const AijItem*)d_items, d_gstart, nitems, ro); break;
+    case OP_AIJ_ONES: hipLaunchKernelGGL(k_aij_ones, ge, dim3(AIJ_THREADS), 0, s, (const AijItem*)d_items, d_gstart, nitems, ro); break;
     case OP_TCG_NT: hipLaunchKernelGGL(k_tcg_nt, ge, te, 0, s, (const TcgItem*)d_items, d_gstart, nitems, ro); break;
     case OP_TCG_RSET: hipLaunchKernelGGL(k_tcg_rset, ge, te, 0, s, (const TcgItem*)d_items, d_gstart, nitems, ro); break;
     case OP_TCG_ZPREP: hipLaunchKernelGGL(k_tcg_zprep, ge, te, 0, s, (const TcgItem*)d_items, d_gstart, nitems, ro); break;
