@@ -3654,14 +3654,19 @@ struct GsbEl {
     double ux, uy;      // s without the row's own changes; s itself once the element is solved
 };
 
-// v of slot `q` (wavefront-uniform) of a register array, lane `l`
+// v of slot `q` (wavefront-uniform) of a register array, lane `l`.  Every slot is read and the
+// values are chosen from: a choice between elements is one between addresses to the compiler, which
+// keeps the array in private memory then, for every other use as well (a call of 33 sweeps on 520 x
+// 24, 14 slots: 794 ms so, 625 ms with the arrays in registers; 262 x 40, four slots: 182 and 163).
 template <int NS>
 __device__ inline double slot_lane(const double (&v)[NS], int q, int l)
 {
     double r = v[0];
 #pragma unroll
-    for (int s = 1; s < NS; s++)
-        if (q == s) r = v[s];
+    for (int s = 1; s < NS; s++) {
+        const double x = v[s];
+        r = q == s ? x : r;
+    }
     return lane_f64(r, l);
 }
 __device__ inline bool uniform_any(bool c) { return __builtin_amdgcn_ballot_w64(c) != 0; }
