@@ -8,6 +8,7 @@
 #include <cmath>
 #include <cstdint>
 #include <cstdio>
+#include <type_traits>
 
 #include "fft_core.hpp"
 #include "ops.hpp"
@@ -3627,24 +3628,36 @@ __global__ void __launch_bounds__(GSB_THREADS) k_gsb_setup(const GsbItem* __rest
     }
 }
 
-// LDS of k_gsb_walk for blocks of `rows` rows: the coefficient rows of the offsets 0 (xx, yy) and
-// 1 .. rows - 1 (xx, xy = yx, yy), each 2 mx; two sets of row elements with their differences at
-// the row's start; and with more than one row the changes of the rows walked and their influence
-// on the next row (two sets, and the four parts of the last row's).
-__host__ __device__ inline size_t gsb_lds_rows(int mx, int rows)
+// LDS of k_gsb_walk for blocks of `rows` rows.  All: the coefficient row of the offset 0 (xx, yy),
+// 2 mx, and two sets of row elements.  With the block's other coefficient rows in the LDS: the
+// offsets 1 .. rows - 1 (xx, xy = yx, yy), each 2 mx; the differences at the start of the two sets'
+// rows; and with more than one row the changes of the rows walked and their influence on the next
+// row (two sets, and the four parts of the last row's).  With the coefficient rows read from memory
+// (wide): the influence of the rows walked, two sets.
+__host__ __device__ inline size_t gsb_lds(int mx, int rows, bool wide)
 {
-    return ((size_t)(4 + 6 * (rows - 1) + 20) + (rows > 1 ? 2 * rows + 12 : 0)) * mx * sizeof(double) +
-           (size_t)4 * rows * sizeof(int) + 64;
+    const size_t cells = wide ? 24 : 24 + 6 * (rows - 1) + (rows > 1 ? 2 * rows + 12 : 0);
+    return cells * mx * sizeof(double) + (size_t)4 * rows * sizeof(int) + 64;
 }
-constexpr int GSB_MAX_ROWS = 8;
-// Rows per block: as many as fit the LDS beside the kernel's static part (0: not even one).  More
-// rows mean fewer products of the whole grid per sweep; those a block holds are summed from LDS.
-__host__ __device__ inline int gsb_fit_rows(int mx)
+constexpr int GSB_MAX_ROWS = 8, GSB_LDS_ROWS = 4;
+// as many rows as fit the LDS beside the kernel's static part (0: not even one)
+__host__ __device__ inline int gsb_fit(int mx, bool wide)
 {
     int r = GSB_MAX_ROWS;
-    while (r > 0 && gsb_lds_rows(mx, r) + 2048 > MAX_LDS) r--;
+    while (r > 0 && gsb_lds(mx, r, wide) + 2048 > MAX_LDS) r--;
     return r;
 }
+// Each block of a sweep costs a product of the whole grid, so that blocks of few rows are dear.  The
+// LDS holds the coefficients of eight rows up to 214 columns, of four up to 325 and of one from 440
+// on; blocks of wider rows keep eight by reading them from memory.  Calls of some forty sweeps on 300
+// rows take, with 300 columns, 2.71 s from the LDS (four rows) and 2.80 from memory; 325: 3.07 (four)
+// and 3.05; 350: 6.8 (three) and 4.2; 450: 16.8 (one) and 7.9; 520: 25.6 (one) and 12.4 s.  On 24 rows
+// of 520 columns 0.63 and 0.31.
+__host__ __device__ inline bool gsb_wide(int mx) { return gsb_fit(mx, false) < GSB_LDS_ROWS; }
+__host__ __device__ inline int gsb_fit_rows(int mx) { return gsb_fit(mx, gsb_wide(mx)); }
+
+template <int N>
+using Count = std::integral_constant<int, N>;
 
 // an element of the row being walked (LDS)
 struct GsbEl {
@@ -3781,13 +3794,9 @@ __device__ __forceinline__ void gsb_walk_row(GsbEl* const row, const double* ear
                                              double eps, double omegah, double omegas)
 {
     const int lane = threadIdx.x & 63;
-    // rows of more than 256 elements read coefficients and bounds where they are used: 14 slots of
-    // them do not fit the registers
-    constexpr bool KEEP = NS <= 4;
-    constexpr int NK = KEEP ? NS : 1;
     double Ux[NS], Uy[NS], Px[NS], Py[NS];
-    double G2[NK];                           // bounds squared
-    GdCell c[NK], l[NK];                     // A(k - ix), A(k - la)
+    double G2[NS];                           // bounds squared
+    GdCell c[NS], l[NS];                     // A(k - ix), A(k - la)
     const GdCell* tk[NS];                    // A(k - 0) of this lane's elements
     auto elem = [&](int s) { return t0 + 64 * s + lane; };
     // (the trailing-edge column has no contact: ConvexGS solves those cases)
@@ -3799,21 +3808,20 @@ __device__ __forceinline__ void gsb_walk_row(GsbEl* const row, const double* ear
         if (early) {
             ux += early[kc];
             uy += early[mx + kc];
-            for (int q = 0; q < 4; q++) {
-                ux += part[2 * q * mx + kc];
-                uy += part[(2 * q + 1) * mx + kc];
-            }
+            if (part)
+                for (int q = 0; q < 4; q++) {
+                    ux += part[2 * q * mx + kc];
+                    uy += part[(2 * q + 1) * mx + kc];
+                }
         }
         Ux[s] = ux;
         Uy[s] = uy;
         Px[s] = row[kc].px;
         Py[s] = row[kc].py;
         tk[s] = tab + kc + mx;
-        if constexpr (KEEP) {
-            G2[s] = row[kc].g * row[kc].g;
-            c[s] = tk[s][-t0];
-            l[s] = tk[s][-la];
-        }
+        G2[s] = row[kc].g * row[kc].g;
+        c[s] = tk[s][-t0];
+        l[s] = tk[s][-la];
     }
     const GdCell b0 = tab[mx], b1 = tab[mx - 1];
     // p of element la (0 in the exterior) and of la + 1
@@ -3828,10 +3836,9 @@ __device__ __forceinline__ void gsb_walk_row(GsbEl* const row, const double* ear
         GsbEl N;
         N.px = row[nx].px; N.py = row[nx].py; N.g = row[nx].g; N.e = row[nx].e; N.dx = row[nx].dx; N.dy = row[nx].dy;
         const GdCell na = tab[la - nx + mx];
-        GdCell nc[NK];
-        if constexpr (KEEP)
+        GdCell nc[NS];
 #pragma unroll
-            for (int s = 0; s < NS; s++) nc[s] = tk[s][-nx];
+        for (int s = 0; s < NS; s++) nc[s] = tk[s][-nx];
         int e = __builtin_amdgcn_readfirstlane((int)E.e);
         if (e >= ADHES) {
             const int q = (ix - t0) >> 6, ol = (ix - t0) & 63;
@@ -3843,16 +3850,8 @@ __device__ __forceinline__ void gsb_walk_row(GsbEl* const row, const double* ear
             dif += Dx * Dx + Dy * Dy;
 #pragma unroll
             for (int s = 0; s < NS; s++) {
-                GdCell ca, cl;
-                if constexpr (KEEP) {
-                    ca = c[s];
-                    cl = l[s];
-                } else {
-                    ca = tk[s][-ix];
-                    cl = tk[s][-la];
-                }
-                Ux[s] = fma(ca.x - cl.x, Dx, Ux[s]);
-                Uy[s] = fma(ca.y - cl.y, Dy, Uy[s]);
+                Ux[s] = fma(c[s].x - l[s].x, Dx, Ux[s]);
+                Uy[s] = fma(c[s].y - l[s].y, Dy, Uy[s]);
                 const bool own = elem(s) == ix;
                 Px[s] = own ? p0 : Px[s];
                 Py[s] = own ? p1 : Py[s];
@@ -3868,16 +3867,9 @@ __device__ __forceinline__ void gsb_walk_row(GsbEl* const row, const double* ear
                     int f = la;              // the first element over its bound, from ix; la: none
 #pragma unroll
                     for (int s = 0; s < NS; s++) {
-                        double g2;
-                        if constexpr (KEEP) {
-                            g2 = G2[s];
-                        } else {
-                            const double g = row[elem(s) <= t1 ? elem(s) : t1].g;
-                            g2 = g * g;
-                        }
                         const double qx = Px[s] + Mx, qy = Py[s] + My;
                         const unsigned long long over = __builtin_amdgcn_ballot_w64(
-                            elem(s) > la && elem(s) < hi && fma(qx, qx, qy * qy) > g2);
+                            elem(s) > la && elem(s) < hi && fma(qx, qx, qy * qy) > G2[s]);
                         if (over) f = t0 + 64 * s + 63 - __clzll((long long)over);
                     }
 #pragma unroll
@@ -3936,14 +3928,12 @@ __device__ __forceinline__ void gsb_walk_row(GsbEl* const row, const double* ear
         if (e != ADHES) {
             la = ix;
             a = b1;
-            if constexpr (KEEP)
 #pragma unroll
-                for (int s = 0; s < NS; s++) l[s] = c[s];
+            for (int s = 0; s < NS; s++) l[s] = c[s];
         }
         E.px = N.px; E.py = N.py; E.g = N.g; E.e = N.e; E.dx = N.dx; E.dy = N.dy;
-        if constexpr (KEEP)
 #pragma unroll
-            for (int s = 0; s < NS; s++) c[s] = nc[s];
+        for (int s = 0; s < NS; s++) c[s] = nc[s];
     }
     difacc += dif;
 #pragma unroll
@@ -3961,27 +3951,26 @@ __device__ __forceinline__ void gsb_walk_row(GsbEl* const row, const double* ear
 // which wavefront 0 adds the row's own changes as it walks (gsb_walk_row).  Meanwhile the other
 // wavefronts read the next row and sum the influence on it of the rows walked before this one;
 // what this row's own change adds to it is summed by all four after the walk.  The block's
-// coefficient rows stay in LDS.  Latency-bound: one wavefront's chain.  With the sum over the row
+// coefficient rows stay in the LDS; those of wide grids are read from memory (WIDE, see gsb_wide),
+// hidden behind the walk but for the last row's.
+// Latency-bound: one wavefront's chain.  With the sum over the row
 // formed for each element, and every row pair's coefficients staged from memory in the gap
 // between two rows, a block of eight rows of a 151 x 97 patch took 1515 us (2.1 us an element),
 // 589 us so; a sweep of an 11 x 11 patch 310 us, 52 us so.
-__global__ void __launch_bounds__(GSB_THREADS) k_gsb_walk(const GsbItem* __restrict__ items, const int* __restrict__ gstart,
-                                                          int nitems, RedOut ro)
+template <bool WIDE>
+__device__ __forceinline__ void gsb_walk_block(const GsbItem& I, double* const lds)
 {
-    extern __shared__ double gsb_lds_[];
-    (void)ro;
-    int it = find_item(gstart, nitems, blockIdx.x);
-    const GsbItem& I = items[it];
     const int mx = I.mx, my = I.my, tid = threadIdx.x, T = blockDim.x, M2 = 2 * mx, wave = tid >> 6;
     const int y0 = I.y0, B = I.y1 - I.y0;
-    GdCell* const tab0 = (GdCell*)gsb_lds_;              // offset 0: (xx, yy)[2 mx], times 1/G
-    double* const tab = gsb_lds_ + 4 * mx;               // [offset - 1][xx, xy, yy][2 mx], times 1/G
-    GsbEl* const els = (GsbEl*)(tab + (size_t)6 * (B - 1) * mx);   // two sets of row elements
+    const bool more = !WIDE && B > 1;
+    GdCell* const tab0 = (GdCell*)lds;                   // offset 0: (xx, yy)[2 mx], times 1/G
+    double* const tab = lds + 4 * mx;                    // [offset - 1][xx, xy, yy][2 mx], times 1/G
+    GsbEl* const els = (GsbEl*)(tab + (WIDE ? (size_t)0 : (size_t)6 * (B - 1) * mx));   // two sets of row elements
     double* const r0 = (double*)(els + 2 * mx);          // two sets [x, y][mx]: differences at the start
-    double* const dd = r0 + 4 * mx;                      // [row][x, y][mx]: changes of the walked rows
-    double* const early = dd + (B > 1 ? 2 * B * mx : 0); // two sets [x, y][mx]: influence of earlier rows
+    double* const dd = r0 + (WIDE ? 0 : 4 * mx);         // [row][x, y][mx]: changes of the walked rows
+    double* const early = dd + (more ? 2 * B * mx : 0);  // two sets [x, y][mx]: influence of earlier rows
     double* const part = early + 4 * mx;                 // four parts [x, y][mx]: of the last row
-    int* const rg = (int*)(early + (B > 1 ? 12 * mx : 0)); // [row][first, last source; first, last interior]
+    int* const rg = (int*)(early + (WIDE ? 4 * mx : more ? 12 * mx : 0)); // [row][first, last source; first, last interior]
     // row t into set b, by threads `first`, first + 1, ...
     auto load_row = [&](int t, int b, int first) {
         const size_t o = (size_t)t * mx;
@@ -3999,8 +3988,10 @@ __global__ void __launch_bounds__(GSB_THREADS) k_gsb_walk(const GsbItem* __restr
             E.ux = wx + zx;
             E.uy = wy + zy;
             els[b * mx + ix] = E;
-            r0[2 * b * mx + ix] = E.dx;
-            r0[(2 * b + 1) * mx + ix] = E.dy;
+            if (!WIDE) {
+                r0[2 * b * mx + ix] = E.dx;
+                r0[(2 * b + 1) * mx + ix] = E.dy;
+            }
         }
     };
     // (ax, ay) += the influence at element k of row n of the changes q0 <= q < q1 of row j
@@ -4018,6 +4009,36 @@ __global__ void __launch_bounds__(GSB_THREADS) k_gsb_walk(const GsbItem* __restr
         ax += sx;
         ay += sy;
     };
+    const double* const cfs[3] = {I.cf[0][0], I.cf[0][1], I.cf[1][1]};   // yx = xy
+    // WIDE: the influence at elements k0 + i step (i < K) of row n of the change of row j, with the
+    // coefficients from memory; change(q, x, y) gives the row's change at element q
+    auto wide_sum = [&](auto K, int k0, int step, int k1, int n, int j, auto change, double* ax, double* ay) {
+        const double* c[3];
+        for (int b = 0; b < 3; b++) c[b] = cfs[b] + (size_t)(my + n - j) * M2 + mx;
+        int at[K];
+#pragma unroll
+        for (int i = 0; i < K; i++) at[i] = min(k0 + i * step, k1);
+        double sx[K], sy[K];
+#pragma unroll
+        for (int i = 0; i < K; i++) sx[i] = sy[i] = 0.0;
+        const int q0 = rg[4 * j], q1 = rg[4 * j + 1];
+#pragma unroll 4
+        for (int q = q0; q <= q1; q++) {
+            double x, y;
+            change(q, x, y);
+#pragma unroll
+            for (int i = 0; i < K; i++) {
+                const double a = as_global(c[1])[at[i] - q];
+                sx[i] = fma(as_global(c[0])[at[i] - q], x, fma(a, y, sx[i]));
+                sy[i] = fma(as_global(c[2])[at[i] - q], y, fma(a, x, sy[i]));
+            }
+        }
+#pragma unroll
+        for (int i = 0; i < K; i++) {
+            ax[i] = fma(I.ga_inv, sx[i], ax[i]);
+            ay[i] = fma(I.ga_inv, sy[i], ay[i]);
+        }
+    };
 
     // d of the previous block has been used by its product: clear it
     for (size_t e = (size_t)I.z0 * mx + tid; e < (size_t)I.z1 * mx; e += T) {
@@ -4025,12 +4046,12 @@ __global__ void __launch_bounds__(GSB_THREADS) k_gsb_walk(const GsbItem* __restr
         as_global(I.ddy)[e] = 0.0;
     }
     for (int e = tid; e < 4 * B; e += T) rg[e] = I.rng[(size_t)(e & 3) * my + y0 + (e >> 2)];
-    const double* const cfs[3] = {I.cf[0][0], I.cf[0][1], I.cf[1][1]};   // yx = xy
     for (int e = tid; e < M2; e += T)
         tab0[e] = GdCell{I.ga_inv * as_global(cfs[0])[(size_t)my * M2 + e], I.ga_inv * as_global(cfs[2])[(size_t)my * M2 + e]};
-    for (int c = 0; c < 3; c++)
-        for (int e = tid; e < (B - 1) * M2; e += T)
-            tab[(size_t)(e / M2 * 3 + c) * M2 + e % M2] = I.ga_inv * as_global(cfs[c])[(size_t)(my + 1) * M2 + e];
+    if (!WIDE)
+        for (int c = 0; c < 3; c++)
+            for (int e = tid; e < (B - 1) * M2; e += T)
+                tab[(size_t)(e / M2 * 3 + c) * M2 + e % M2] = I.ga_inv * as_global(cfs[c])[(size_t)(my + 1) * M2 + e];
     __syncthreads();
     // the next row with an interior element, or B
     auto next_row = [&](int r) {
@@ -4050,23 +4071,58 @@ __global__ void __launch_bounds__(GSB_THREADS) k_gsb_walk(const GsbItem* __restr
         if (wave == 0) {
             const int nt = t1 - t0 + 1;
             const double* ev = first ? nullptr : early + 2 * b * mx;
-            if (nt <= 64) gsb_walk_row<1>(row, ev, part, mx, t0, t1, tab0, difacc, I.eps, I.omegah, I.omegas);
-            else if (nt <= 128) gsb_walk_row<2>(row, ev, part, mx, t0, t1, tab0, difacc, I.eps, I.omegah, I.omegas);
-            else if (nt <= 256) gsb_walk_row<4>(row, ev, part, mx, t0, t1, tab0, difacc, I.eps, I.omegah, I.omegas);
-            else gsb_walk_row<14>(row, ev, part, mx, t0, t1, tab0, difacc, I.eps, I.omegah, I.omegas);
+            const double* pt = WIDE ? nullptr : part;
+            auto walk = [&](auto ns) {
+                gsb_walk_row<ns>(row, ev, pt, mx, t0, t1, tab0, difacc, I.eps, I.omegah, I.omegas);
+            };
+            // slots of 64 elements, few of them beyond the row's end (each costs every element some
+            // 50 cycles); of the rows that the LDS form takes none has more than 325 elements
+            if constexpr (WIDE) {
+                if (nt <= 256) walk(Count<4>());
+                else if (nt <= 384) walk(Count<6>());
+                else if (nt <= 512) walk(Count<8>());
+                else if (nt <= 704) walk(Count<11>());
+                else walk(Count<14>());
+            } else {
+                if (nt <= 64) walk(Count<1>());
+                else if (nt <= 128) walk(Count<2>());
+                else if (nt <= 256) walk(Count<4>());
+                else walk(Count<6>());
+            }
             flops += 4.0 * nt * nt;
         } else if (n < B) {
             load_row(y0 + n, b ^ 1, 64);
             // the influence on row n of the rows walked before this one
             double* const ev = early + 2 * (b ^ 1) * mx;
-            for (int k = rg[4 * n + 2] + tid - 64; k <= rg[4 * n + 3]; k += T - 64) {
-                double ax = 0.0, ay = 0.0;
-                for (int j = 0; j < r; j++) {
-                    if (rg[4 * j + 3] < rg[4 * j + 2]) continue;
-                    row_sum(k, n, j, rg[4 * j], rg[4 * j + 1] + 1, ax, ay);
+            const int k1 = rg[4 * n + 3];
+            if constexpr (WIDE) {
+                constexpr int K = 3;
+                for (int k0 = rg[4 * n + 2] + tid - 64; k0 <= k1; k0 += K * (T - 64)) {
+                    double ax[K] = {}, ay[K] = {};
+                    for (int j = 0; j < r; j++) {
+                        if (rg[4 * j + 3] < rg[4 * j + 2]) continue;
+                        const size_t o = (size_t)(y0 + j) * mx;
+                        wide_sum(Count<K>(), k0, T - 64, k1, n, j, [&](int q, double& x, double& y) {
+                            x = as_global(I.ddx)[o + q];
+                            y = as_global(I.ddy)[o + q];
+                        }, ax, ay);
+                    }
+                    for (int i = 0; i < K; i++)
+                        if (k0 + i * (T - 64) <= k1) {
+                            ev[k0 + i * (T - 64)] = ax[i];
+                            ev[mx + k0 + i * (T - 64)] = ay[i];
+                        }
                 }
-                ev[k] = ax;
-                ev[mx + k] = ay;
+            } else {
+                for (int k = rg[4 * n + 2] + tid - 64; k <= k1; k += T - 64) {
+                    double ax = 0.0, ay = 0.0;
+                    for (int j = 0; j < r; j++) {
+                        if (rg[4 * j + 3] < rg[4 * j + 2]) continue;
+                        row_sum(k, n, j, rg[4 * j], rg[4 * j + 1] + 1, ax, ay);
+                    }
+                    ev[k] = ax;
+                    ev[mx + k] = ay;
+                }
             }
         }
         __syncthreads();
@@ -4078,7 +4134,8 @@ __global__ void __launch_bounds__(GSB_THREADS) k_gsb_walk(const GsbItem* __restr
                 as_global(I.sx)[o + ix] = E.ux;
                 as_global(I.sy)[o + ix] = E.uy;
             }
-            const double cx = E.dx - r0[2 * b * mx + ix], cy = E.dy - r0[(2 * b + 1) * mx + ix];
+            const double cx = E.dx - (WIDE ? as_global(I.dpx)[o + ix] : r0[2 * b * mx + ix]);
+            const double cy = E.dy - (WIDE ? as_global(I.dpy)[o + ix] : r0[(2 * b + 1) * mx + ix]);
             as_global(I.px)[o + ix] = E.px;
             as_global(I.py)[o + ix] = E.py;
             as_global(I.dpx)[o + ix] = E.dx;
@@ -4086,16 +4143,41 @@ __global__ void __launch_bounds__(GSB_THREADS) k_gsb_walk(const GsbItem* __restr
             as_global(I.ddx)[o + ix] = cx;
             as_global(I.ddy)[o + ix] = cy;
             as_global(I.el)[o + ix] = (int8_t)E.e;
-            if (B > 1) {
+            if (WIDE) {
+                row[ix].dx = cx;
+                row[ix].dy = cy;
+            } else if (more) {
                 dd[(size_t)2 * r * mx + ix] = cx;
                 dd[(size_t)(2 * r + 1) * mx + ix] = cy;
             }
         }
         if (n >= B) break;
         __syncthreads();
-        // the influence on row n of this row's change, a part of the sum by each wavefront
-        {
-            const int q0 = rg[4 * r], nq = rg[4 * r + 1] + 1 - q0, per = (nq + 3) / 4;
+        // the influence on row n of this row's change: an element or two of the row by each thread,
+        // or a part of the sum by each wavefront
+        const int nq = rg[4 * r + 1] + 1 - rg[4 * r];
+        if constexpr (WIDE) {
+            constexpr int K = 2;
+            double* const ev = early + 2 * (b ^ 1) * mx;
+            const int k1 = rg[4 * n + 3];
+            for (int k0 = rg[4 * n + 2] + tid; k0 <= k1; k0 += K * T) {
+                double ax[K], ay[K];
+                for (int i = 0; i < K; i++) {
+                    ax[i] = k0 + i * T <= k1 ? ev[k0 + i * T] : 0.0;
+                    ay[i] = k0 + i * T <= k1 ? ev[mx + k0 + i * T] : 0.0;
+                }
+                wide_sum(Count<K>(), k0, T, k1, n, r, [&](int q, double& x, double& y) {
+                    x = row[q].dx;
+                    y = row[q].dy;
+                }, ax, ay);
+                for (int i = 0; i < K; i++)
+                    if (k0 + i * T <= k1) {
+                        ev[k0 + i * T] = ax[i];
+                        ev[mx + k0 + i * T] = ay[i];
+                    }
+            }
+        } else {
+            const int q0 = rg[4 * r], per = (nq + 3) / 4;
             const int qa = q0 + min(nq, wave * per), qb = q0 + min(nq, (wave + 1) * per);
             for (int k = rg[4 * n + 2] + (tid & 63); k <= rg[4 * n + 3]; k += 64) {
                 double ax = 0.0, ay = 0.0;
@@ -4103,8 +4185,8 @@ __global__ void __launch_bounds__(GSB_THREADS) k_gsb_walk(const GsbItem* __restr
                 part[2 * wave * mx + k] = ax;
                 part[(2 * wave + 1) * mx + k] = ay;
             }
-            if (tid == 0) flops += 8.0 * nq * (rg[4 * n + 3] - rg[4 * n + 2] + 1) * (r + 1);
         }
+        if (tid == 0) flops += 8.0 * nq * (rg[4 * n + 3] - rg[4 * n + 2] + 1) * (r + 1);
         __syncthreads();
         r = n;
         b ^= 1;
@@ -4114,6 +4196,16 @@ __global__ void __launch_bounds__(GSB_THREADS) k_gsb_walk(const GsbItem* __restr
         I.st[0] += difacc;
         I.st[3] += flops;
     }
+}
+
+__global__ void __launch_bounds__(GSB_THREADS) k_gsb_walk(const GsbItem* __restrict__ items, const int* __restrict__ gstart,
+                                                          int nitems, RedOut ro)
+{
+    extern __shared__ double gsb_lds_[];
+    (void)ro;
+    const GsbItem& I = items[find_item(gstart, nitems, blockIdx.x)];
+    if (gsb_wide(I.mx)) gsb_walk_block<true>(I, gsb_lds_);
+    else gsb_walk_block<false>(I, gsb_lds_);
 }
 
 // end of a sweep (src/m_solvpt.f90:3130-3150): dif = sqrt(sum |dp|^2 / 2k), difid from the rms
@@ -4696,7 +4788,10 @@ double op_bytes(int kind, const void* item, int stage)
 size_t op_lds(int kind, const void* item, int stage)
 {
     if (kind == OP_CONV || kind == OP_CONV32) return conv_lds(kind, (const ConvItem*)item, stage);
-    if (kind == OP_GSB_WALK) return gsb_lds_rows(((const GsbItem*)item)->mx, ((const GsbItem*)item)->y1 - ((const GsbItem*)item)->y0);
+    if (kind == OP_GSB_WALK) {
+        const GsbItem* g = (const GsbItem*)item;
+        return gsb_lds(g->mx, g->y1 - g->y0, gsb_wide(g->mx));
+    }
     if (kind == OP_GD_PROJECT || kind == OP_GD_PROBE || kind == OP_GD_UPDATE) {
         const GdItem* g = (const GdItem*)item;
         int R = gd_rows_per_tile(g->mx, g->my, gd_tile(kind));
@@ -4705,7 +4800,7 @@ size_t op_lds(int kind, const void* item, int stage)
     }
     if (kind == OP_STDYGS) {
         const GsItem* g = (const GsItem*)item;
-        if (stage == 3) return g->mx >= 2 ? gsb_lds_rows(g->mx, 1) : MAX_LDS + 1;   // rng needs 4 my <= 2 n
+        if (stage == 3) return g->mx >= 2 ? gsb_lds(g->mx, 1, gsb_wide(g->mx)) : MAX_LDS + 1;   // rng needs 4 my <= 2 n
         if (stage == 2) return gs3_lds(g->mx, g->my);
         if (stage == 1) return gs2_lds(g->mx, g->my);
         return (size_t)g->mx * (5 * sizeof(double) + 1) + (size_t)(2 * g->my + 1) * sizeof(int) + 16;

@@ -346,6 +346,7 @@ struct orc_problem {
     int ierror;
     int gd_stagnated;
     int used_stdygs;
+    long gs_clips;      /* SteadyGS: upstream elements put on their bound */
     int use_cnvxgs;     /* the tangential solver of this case is ConvexGS (set by stang) */
     /* sensitivities sens(iout, iin), column-major as in the reference (outpt%sens) */
     double sens[16];
@@ -1912,6 +1913,7 @@ static int stdygs(orc_problem *P, double **ws, const double *mus, int k, double 
                         if (ptabs > ptbnd) {
                             px[jj] = px[jj] * ptbnd / ptabs;
                             py[jj] = py[jj] * ptbnd / ptabs;
+                            P->gs_clips++;
                             dpx[jj] = px[jj] - px[jn];
                             dpy[jj] = py[jj] - py[jn];
                         }
@@ -2772,6 +2774,7 @@ int orc_calculate(orc_problem *P, const orc_input *inp)
     P->itnorm = P->ittang = P->itcg = P->itgs = 0;
     P->gd_stagnated = 0;
     P->used_stdygs = 0;
+    P->gs_clips = 0;
     if (inp->tang < 0 || inp->tang > 3) return P->ierror = CNTC_ERR_OTHER;
     /* combin_mater, src/m_hierarch_data.f90:1543-1553 */
     P->ga = 2.0 / (1.0 / inp->gg1 + 1.0 / inp->gg2);
@@ -3084,6 +3087,7 @@ void orc_get_iters(const orc_problem *p, int *itnorm, int *ittang, int *itcg, in
 {
     *itnorm = p->itnorm; *ittang = p->ittang; *itcg = p->itcg; *itgs = p->itgs;
 }
+long orc_get_gs_clips(const orc_problem *p) { return p->gs_clips; }
 int orc_get_stagnated(const orc_problem *p) { return p->gd_stagnated + 2 * p->used_stdygs; }
 void orc_get_sens(const orc_problem *p, double *sens) { memcpy(sens, p->sens, sizeof p->sens); }
 void orc_get_creepages(const orc_problem *p, double *cksi, double *ceta, double *cphi)

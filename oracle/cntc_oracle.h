@@ -106,6 +106,9 @@ void orc_get_iters(const orc_problem *p, int *itnorm, int *ittang, int *itcg, in
 /* bit 0: the last GDsteady call ended in stagnation (src/gdsteady.f90:560-585);
    bit 1: SteadyGS ran in the last case */
 int  orc_get_stagnated(const orc_problem *p);
+/* adhesion elements that SteadyGS put on their bound while it rebuilt the upstream part of a row
+   (src/m_solvpt.f90:3086-3127), in the last case */
+long orc_get_gs_clips(const orc_problem *p);
 /* sensitivity matrix in internal units, sens[iout + 4*iin] with outputs (fn, fx/(mu fn),
    fy/(mu fn), mz) and inputs (pen, cksi, ceta, cphi), src/m_hierarch_data.f90:122-124 */
 void orc_get_sens(const orc_problem *p, double *sens);

@@ -80,6 +80,8 @@ def lib():
         L.orc_get_iters.argtypes = [vp, ip, ip, ip, ip]
         L.orc_get_stagnated.argtypes = [vp]
         L.orc_get_stagnated.restype = ctypes.c_int
+        L.orc_get_gs_clips.argtypes = [vp]
+        L.orc_get_gs_clips.restype = ctypes.c_long
         L.orc_get_sens.argtypes = [vp, dp]
         L.orc_get_creepages.argtypes = [vp, dp, dp, dp]
         L.orc_linrol.argtypes = [ctypes.c_double, ctypes.c_double, dp, dp, dp]
@@ -179,6 +181,10 @@ class Problem:
 
     def stagnated(self):
         return lib().orc_get_stagnated(self._p)
+
+    def gs_clips(self):
+        """Upstream adhesion elements that SteadyGS put on their bound in the last case."""
+        return lib().orc_get_gs_clips(self._p)
 
     def sens(self):
         """4x4 sensitivities in internal units, [iout, iin]: outputs (fn, fx/(mu fn),

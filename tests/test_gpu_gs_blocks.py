@@ -36,3 +36,36 @@ def test_row_widths(cntc, oracle, mx, my, gausei):
         assert np.abs(a - b).max() <= 1e-7 * np.abs(P.tractions()[0]).max()
     for a, b in zip(f[:3], of[:3]):
         assert abs(a - b) <= 1e-7 * c["fstat"] * c["fn"]
+
+
+# mx, my, elements that the widest row has to exceed: coefficients in the LDS for blocks of 7, 5 and 4
+# rows; read from memory for rows that take 6, 8, 11 and 14 slots, in blocks of 8 rows with a second
+# one of 5, 1 and none, and of 4 on the widest grid that blocks take
+WIDE = [(220, 12, 128), (288, 10, 256), (325, 9, 256), (326, 13, 256), (420, 9, 384), (560, 8, 512), (842, 8, 704)]
+
+
+@pytest.mark.parametrize("mx,my,wider", WIDE)
+def test_wide_rows(cntc, oracle, mx, my, wider):
+    """The same sweeps as the oracle, cut off at eps 1e-3: an element's problem is solved to 1e-4 eps of
+    its bound, which some 50 sweeps add up to 5e-6 of mu p at worst: compared to 1e-5 of the largest
+    pressure and of mu Fn.  Elements upstream have to be put on their bound on the way."""
+    c = W.base_case(tang=3, norm=1, fn=9e4 * my / mx, cksi=-3e-4, ceta=1e-4, cphi=1e-4, eps=1e-3, ipotcn=-3, mx=mx,
+                    my=my, aa=6.0, bb=6.0 * my / mx, scale=mx / (mx - 4.0), gausei=0)
+    rc, of, P = oracle.solve_case(c)
+    assert rc == 0
+    ire = 944
+    W.apply_case(cntc, ire, 1, c)
+    assert cntc.calculate(ire, 1) == 0
+    p = [a.ravel() for a in cntc.gettractions(ire, 1)]
+    f, its = cntc.getcontactforces(ire, 1), cntc.getiterations(ire, 1)
+    el = cntc.getelementdivision(ire, 1).reshape(my, mx)
+    cntc.finalize(ire)
+    inside = (el > 0).sum(1)
+    print(mx, my, "widest row", inside.max(), "rows", (inside > 0).sum(), "iterations", its, P.iters(), "clips", P.gs_clips())
+    assert its[4] & 2 and its[3] == P.iters()[3]
+    assert inside.max() > wider and inside.min() > 0
+    assert P.gs_clips() > 100
+    for a, b in zip(p, P.tractions()):
+        assert np.abs(a - b).max() <= 1e-5 * np.abs(P.tractions()[0]).max()
+    for a, b in zip(f[:3], of[:3]):
+        assert abs(a - b) <= 1e-5 * c["fstat"] * c["fn"]

@@ -35,6 +35,14 @@ def test_exported_symbols_are_plain_c(cntc):
         assert n in exported, n
 
 
+def test_steadygs_rows_per_block(cntc):
+    """SteadyGS by blocks: a product of the whole grid per block, so no block of a few rows, as far as
+    the widest grid whose rows fit the LDS."""
+    rows = getattr(ctypes.CDLL(cntc.library_path), "_ZN4cntc14gsb_block_rowsEi")
+    assert [rows(mx) for mx in (11, 214, 215, 325, 326, 440, 668, 841)] == [8, 8, 7, 4, 8, 8, 8, 8]
+    assert all(rows(mx) >= 4 for mx in range(2, 843)) and rows(843) == 0
+
+
 @pytest.mark.skipif(os.path.exists("/dev/kfd"), reason="a GPU is present")
 def test_calculate_without_gpu_fails_loudly(cntc):
     """No CPU fallback: without a GPU the solve reports CNTC_err_other."""
