@@ -851,9 +851,9 @@ __host__ __device__ inline int gd_rows_per_tile(int mx, int my, int tile)
 __host__ __device__ inline int gd_row_stride(int mx) { return mx | 1; }
 
 // Cells of the LDS tiles of the row recurrences: two components side by side; and for
-// apply_trcbnd the bound with the state in its sign (adhesion g, slip -g, exterior +inf; GD has
-// no other states) and the least |p|^2 at which the bound has to be looked at (in adhesion
-// below g^2 by more than the rounding of a square root: p2 < lim implies sqrt(p2) < g).
+// apply_trcbnd the bound g, of either sign, and the least |p|^2 at which it has to be looked at (in
+// adhesion below g^2 by more than the rounding of a square root: p2 < lim implies sqrt(p2) < g).
+// The state is in lim: slip -1, exterior +inf, adhesion finite (GD has no other states).
 struct GdCell {
     double x, y;
 };
@@ -862,12 +862,12 @@ struct GdBound {
 };
 __device__ inline GdBound gd_bound(double g, int8_t st)
 {
-    if (st == ADHES) return GdBound{g, g * g * (1.0 - 0x1p-50)};
-    return st == SLIP ? GdBound{-g, -1.0} : GdBound{INFINITY, INFINITY};
+    if (st == ADHES) return GdBound{g, g > 0.0 ? fmin(g * g * (1.0 - 0x1p-50), 0x1.fffffffffffffp1023) : 0.0};
+    return st == SLIP ? GdBound{g, -1.0} : GdBound{g, INFINITY};
 }
 __device__ inline int8_t gd_state(const GdBound& b)
 {
-    return b.c == INFINITY ? EXTER : (b.lim < 0.0 ? SLIP : ADHES);
+    return b.lim == INFINITY ? EXTER : (b.lim < 0.0 ? SLIP : ADHES);
 }
 
 // apply_trcbnd along one row (src/gdsteady.f90:807-847): from the leading edge, p = p(ix+1) + dp,
@@ -894,11 +894,12 @@ __device__ inline void trcbnd_row(GdCell* lp, const GdBound* lb, int mx)
         const double p2 = fma(px, px, py * py);
         const bool need = !(p2 < b.lim);
         if (__builtin_amdgcn_ballot_w64(need)) {
-            const double g = fabs(b.c), nx = px * g, ny = py * g;
+            const double nx = px * b.c, ny = py * b.c;
+            const bool slip = b.lim < 0.0;
             const bool wide = (unsigned)(__double2hiint(p2) - (423 << 20)) >= (1200u << 20);
             if (__builtin_amdgcn_ballot_w64(need && wide)) {
                 const double s = sqrt(p2);
-                if (need && s >= b.c) {
+                if (need && (slip || s >= b.c)) {
                     px = nx / s;
                     py = ny / s;
                 }
@@ -913,14 +914,14 @@ __device__ inline void trcbnd_row(GdCell* lp, const GdBound* lb, int mx)
                 double q = h + h;
                 q = fma(q, fma(-s, q, 1.0), q);
                 const double qx = nx * q, qy = ny * q;
-                const bool clip = s >= b.c;   // (true in slip, false in the exterior)
+                const bool clip = slip || s >= b.c;
                 const double ex = copysign(fma(fma(-s, qx, nx), q, qx), nx);
                 const double ey = copysign(fma(fma(-s, qy, ny), q, qy), ny);
                 px = clip ? ex : px;
                 py = clip ? ey : py;
             }
         }
-        const bool ext = __double2hiint(b.c) == 0x7FF00000;
+        const bool ext = __double2hiint(b.lim) == 0x7FF00000;
         pxn = ext ? 0.0 : px;
         pyn = ext ? 0.0 : py;
         lp[ix] = GdCell{pxn, pyn};
@@ -1253,7 +1254,7 @@ __global__ void __launch_bounds__(T, 4) k_gd_probe(const GdItem* __restrict__ it
         GdBound d{0.0, 0.0};
         if (st == ADHES || st == SLIP) {
             double sx = t.sx, sy = t.sy, qx = t.qx, qy = t.qy;
-            double px = lp[l].x, py = lp[l].y, g = fabs(b.c);
+            double px = lp[l].x, py = lp[l].y, g = b.c;
             double txo = -t.ny, tyo = t.nx;
             double vt = t.vx * txo + t.vy * tyo;
             double dth_da = (g * vt) / (fmax(tiny, g * g) + a * a * vt * vt);
@@ -1454,12 +1455,12 @@ __device__ void elmtrc(int8_t& el, const double c11, const double c12, const dou
             pr[0] = pold1 + omegah * dp0;
             pr[1] = pold2 + omegah * dp1;
             const double p2 = pr[0] * pr[0] + pr[1] * pr[1];
-            const double bnd = fmin(trc_bound, taucs);
-            if (p2 <= bnd * bnd) {
+            const double bnd = fmin(trc_bound, taucs), b2 = bnd * fabs(bnd);
+            if (p2 <= b2) {
                 violat = 0;
             } else {
                 const double q0 = pold1 + dp0, q1 = pold2 + dp1;
-                if (q0 * q0 + q1 * q1 <= bnd * bnd) {
+                if (q0 * q0 + q1 * q1 <= b2) {
                     const double f = bnd * fast_rsqrt(p2);
                     pr[0] *= f;
                     pr[1] *= f;
@@ -3711,7 +3712,7 @@ __device__ inline void elmtrc_uniform(int& el, double c11, double c22, double ep
             const double d0 = -in0 * fast_rcp(stay_here(c11)), d1 = -in1 * fast_rcp(stay_here(c22));
             p0 = fma(omegah, d0, o0);
             p1 = fma(omegah, d1, o1);
-            const double p2 = fma(p0, p0, p1 * p1), bnd = fmin(tb, 1e20), b2 = bnd * bnd;
+            const double p2 = fma(p0, p0, p1 * p1), bnd = fmin(tb, 1e20), b2 = bnd * fabs(bnd);
             violat = false;
             if (uniform_any(!(p2 <= b2))) {
                 const double q0 = o0 + d0, q1 = o1 + d1;
@@ -3795,7 +3796,7 @@ __device__ __forceinline__ void gsb_walk_row(GsbEl* const row, const double* ear
 {
     const int lane = threadIdx.x & 63;
     double Ux[NS], Uy[NS], Px[NS], Py[NS];
-    double G2[NS];                           // bounds squared
+    double G2[NS];                           // bounds squared, with their sign
     GdCell c[NS], l[NS];                     // A(k - ix), A(k - la)
     const GdCell* tk[NS];                    // A(k - 0) of this lane's elements
     auto elem = [&](int s) { return t0 + 64 * s + lane; };
@@ -3819,7 +3820,7 @@ __device__ __forceinline__ void gsb_walk_row(GsbEl* const row, const double* ear
         Px[s] = row[kc].px;
         Py[s] = row[kc].py;
         tk[s] = tab + kc + mx;
-        G2[s] = row[kc].g * row[kc].g;
+        G2[s] = row[kc].g * fabs(row[kc].g);
         c[s] = tk[s][-t0];
         l[s] = tk[s][-la];
     }
