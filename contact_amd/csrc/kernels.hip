@@ -3693,11 +3693,10 @@ __device__ inline double stay_here(double x)
 }
 
 // elmtrc (src/m_solvpt.f90:3258-3807) on the latency path: the steps of elmtrc with scale_dir,
-// on data that every lane holds alike, so that its branches are scalar.  c12 = c21 = 0: within a
-// row the xy coefficients vanish by symmetry (the tables hold their rounding, 1e-17 of xx).  The
-// iterates are those of elmtrc: the Newton corrections divide through a once refined reciprocal
-// (good to 2^-45 of a correction), the starting direction through a once refined reciprocal
-// square root.
+// on data that every lane holds alike, so that its branches are scalar, with its iterates: divisions
+// and square roots through the same refined reciprocals.  c12 = c21 = 0: within a row the xy
+// coefficients of a half space vanish by symmetry (the tables hold their rounding, below 1e-15 of
+// xx).  Coefficients without that symmetry need the xy terms here and in gsb_walk_row.
 __device__ inline void elmtrc_uniform(int& el, double c11, double c22, double eps, double& p0, double& p1,
                                       double tb, double& s0, double& s1, double omegah, double omegas)
 {
@@ -3728,8 +3727,7 @@ __device__ inline void elmtrc_uniform(int& el, double c11, double c22, double ep
             siy = fma(c22, p1, si0y);
         } else if (el == SLIP) {
             const double bx = stay_here(si0x), by = stay_here(si0y);
-            const double a2 = fma(bx, bx, by * by), y = __builtin_amdgcn_rsq(a2);
-            const double f = -tb * fma(y, fma(-0.5 * a2 * y, y, 0.5), y);
+            const double f = -tb * fast_rsqrt(fma(bx, bx, by * by));
             p0 = f * bx;
             p1 = f * by;
             const double tb2 = tb * tb, dc = c11 - c22, lim = prc * eps * tb;
@@ -3741,9 +3739,7 @@ __device__ inline void elmtrc_uniform(int& el, double c11, double c22, double ep
                 const double g10 = 2.0 * p0, g11 = 2.0 * p1;
                 const double det = fma(g00, g11, -(g01 * g10));
                 const double n0 = fma(g01, fk1, -(g11 * fk0)), n1 = fma(g10, fk0, -(g00 * fk1));
-                double r = __builtin_amdgcn_rcp(det);
-                r = fma(r, fma(-det, r, 1.0), r);
-                r = det == 0.0 ? 0.0 : r;      // (no correction then, as in elmtrc)
+                const double r = det == 0.0 ? 0.0 : fast_rcp(det);   // (0: no correction, as in elmtrc)
                 p0 = fma(n0, r, p0);
                 p1 = fma(n1, r, p1);
                 six = fma(c11, p0, bx);
