@@ -837,7 +837,7 @@ __global__ void __launch_bounds__(ELEM_THREADS) k_st_sa(const StItem* __restrict
 // recurrence in LDS, and the element-wise rest is done by all threads with coalesced access.
 constexpr int GD_THREADS = 256;
 constexpr int GD_ROW_THREADS = 256;    // threads of project
-constexpr int GD_ELEM_THREADS = ELEM_THREADS * ELEM_PER_THREAD;   // an element per thread
+constexpr int GD_ELEM_TILE = ELEM_THREADS * ELEM_PER_THREAD;   // elements per group (moves, diagres)
 constexpr int GD_TILE = 2048;          // elements per tile (probe; its sums follow this shape)
 constexpr int GD_TILE_ROW = 1024;      // elements per tile (update, project)
 
@@ -1573,12 +1573,12 @@ __device__ void elmtrc(int8_t& el, const double c11, const double c12, const dou
 // follow from its solution are used, so it is solved on the latency path (elmtrc, scale_dir).
 // With four elements in turn and the general problem 20.3 us a launch for a mix of sides 20 to 256,
 // 10.1 us so; 1024 x 1024 33.2 and 26.5 us (HIP events, about 4 us of each their own).
-__global__ void __launch_bounds__(GD_ELEM_THREADS) k_gd_moves(const GdItem* __restrict__ items, const int* __restrict__ gstart,
+__global__ void __launch_bounds__(GD_ELEM_TILE) k_gd_moves(const GdItem* __restrict__ items, const int* __restrict__ gstart,
                                                               int nitems, RedOut ro)
 {
     int it = find_item(gstart, nitems, blockIdx.x);
     const GdItem& I = items[it];
-    const int i = (blockIdx.x - gstart[it]) * GD_ELEM_THREADS + threadIdx.x;
+    const int i = (blockIdx.x - gstart[it]) * GD_ELEM_TILE + threadIdx.x;
     double acc[1] = {0.0};
     const double tiny = 1e-12;
     const size_t ii = i < I.n ? i : 0;
@@ -1645,101 +1645,109 @@ __device__ inline bool gd_slip_split(const GdItem& I, const double px, const dou
 
 // compute_diagscaling and the scaled residual (src/gdsteady.f90:901-1042, 429-439); when
 // not I.first also pold -= p on the interior.  Returns (sum (pold)^2, sum p^2, sum_int r^2).
-// An element per thread: latency-bound by the slip elements' angles and 2x2 problem.  The start
-// of an element's run of adhesion is found from the states of the wavefront, 64 at a time.  The
-// sums are those of 256 threads with elements t, t + 256, ... each.  With four elements in turn and the run walked element by element 43.4 us a launch for a
-// mix of sides 20 to 256, 20.2 us so; 40 x 40 29.6 and 18.6, 1024 x 1024 65.7 and 73.5 us (HIP
-// events, about 4 us of each their own).
-__global__ void __launch_bounds__(GD_ELEM_THREADS) k_gd_diagres(const GdItem* __restrict__ items, const int* __restrict__ gstart,
-                                                                int nitems, RedOut ro)
+// Latency-bound by the slip elements' angles and 2x2 problem: an element per thread while every group
+// has a compute unit to itself.  With more groups 256 threads take four elements in turn: two groups
+// share a compute unit then, without spilling (195 registers), and none waits for the slowest of 1024
+// threads.  The start of an element's run of adhesion is found from the states of the wavefront, 64 at
+// a time.  The sums are those of 256 threads with elements t, t + 256, ... each.  Four elements in turn
+// and the run walked element by element / 1024 threads / 256: 40 x 40 28.6, 18.1, 23.7 us a launch; 48
+// patches of sides 20 to 72 51.9, 19.6, 31.6; 512 x 512 (256 groups) 39.4, 24.2, 29.4; 1024 x 1024
+// 94.5, 73.5, 56.6 (HIP events, about 4 us of each their own).
+template <int T>
+__global__ void __launch_bounds__(T, T == 1024 ? 4 : 2) k_gd_diagres(const GdItem* __restrict__ items, const int* __restrict__ gstart,
+                                                                     int nitems, RedOut ro)
 {
-    __shared__ double con[3][GD_ELEM_THREADS];
+    __shared__ double con[3][GD_ELEM_TILE];
     int it = find_item(gstart, nitems, blockIdx.x);
     const GdItem& I = items[it];
-    const int mx = I.mx, i = (blockIdx.x - gstart[it]) * GD_ELEM_THREADS + threadIdx.x;
-    const bool in = i < I.n;
-    const size_t ii = in ? i : 0;
-    const int8_t s = in ? as_global(I.el)[ii] : EXTER;
-    const double px = as_global(I.px)[ii], py = as_global(I.py)[ii], pn = as_global(I.pn)[ii];
-    const double sx = as_global(I.sx)[ii], sy = as_global(I.sy)[ii];
-    const double nx = as_global(I.nx)[ii], ny = as_global(I.ny)[ii];
-    double ox = 0.0, oy = 0.0;
-    if (!I.first) {
-        ox = as_global(I.poldx)[ii];
-        oy = as_global(I.poldy)[ii];
-    }
-    double dscl = as_global(I.dscl)[ii];
-    // the run of adhesion that this element ends: its first element is the nearest one, at or
-    // before this one, that begins the row or follows an element not in adhesion
-    auto begins = [&](int j) { return j % mx == 0 || as_global(I.el)[j - 1] != ADHES; };
-    const int lane = threadIdx.x & 63, w0 = i - lane;
-    const unsigned long long stop = __builtin_amdgcn_ballot_w64(!in || begins(i));
-    const unsigned long long mine = stop & (~0ull >> (63 - lane));
-    int start = w0 + 63 - __clzll((long long)mine);
-    if (!(stop & 1)) {
-        int prev = 0;
-        for (int c = w0 - 64; c >= 0; c -= 64) {
-            const unsigned long long b = __builtin_amdgcn_ballot_w64(begins(c + lane));
-            if (b) {
-                prev = c + 63 - __clzll((long long)b);
-                break;
-            }
-        }
-        if (!mine) start = prev;
-    }
-    double rx = 0.0, ry = 0.0, c0 = 0.0, c1 = 0.0, c2 = 0.0;
-    if (in) {
-        int8_t elnew = EXTER;
-        double fac_s = 0.0;
-        bool have = false;
-        if (s == SLIP) have = gd_slip_split(I, px, py, pn, sx, sy, elnew, fac_s);
-        if (s == SLIP && !have) {
-            // the reference keeps elnew/fac_s of the last slip element it split
-            for (int j = i - 1; j >= 0; j--) {
-                if (I.el[j] != SLIP) continue;
-                if (gd_slip_split(I, I.px[j], I.py[j], I.pn[j], I.sx[j], I.sy[j], elnew, fac_s)) break;
-            }
-        }
-        if (s == SLIP && elnew == SLIP) {
-            dscl = I.d_slp * pow(fac_s, I.pow_s);
-        } else if (s == ADHES || (s == SLIP && elnew == ADHES)) {
-            const int run = i - start;
-            double dnew;
-            if (I.d_cns < I.d_ifc)
-                dnew = fmax(I.d_cns, I.d_ifc + (run - 1) * fmin(0.0, I.d_lin));
-            else
-                dnew = fmin(I.d_cns, I.d_ifc + (run - 1) * fmax(0.0, I.d_lin));
-            dscl = fmin(50.0 * dscl, dnew);
-        } else if (s != ADHES) {
-            dscl = 0.0;
-        }
-        as_global(I.dscl)[ii] = dscl;
-        if (s == ADHES) {
-            rx = -sx * dscl;
-            ry = -sy * dscl;
-        } else if (s == SLIP) {
-            double tx = -ny, ty = nx;
-            double st = tx * sx + ty * sy;
-            rx = -st * tx * dscl;
-            ry = -st * ty * dscl;
-        }
-        as_global(I.rx)[ii] = rx;
-        as_global(I.ry)[ii] = ry;
+    const int mx = I.mx;
+#pragma unroll 1
+    for (int own = threadIdx.x; own < GD_ELEM_TILE; own += T) {
+        const int i = (blockIdx.x - gstart[it]) * GD_ELEM_TILE + own;
+        const bool in = i < I.n;
+        const size_t ii = in ? i : 0;
+        const int8_t s = in ? as_global(I.el)[ii] : EXTER;
+        const double px = as_global(I.px)[ii], py = as_global(I.py)[ii], pn = as_global(I.pn)[ii];
+        const double sx = as_global(I.sx)[ii], sy = as_global(I.sy)[ii];
+        const double nx = as_global(I.nx)[ii], ny = as_global(I.ny)[ii];
+        double ox = 0.0, oy = 0.0;
         if (!I.first) {
-            if (s >= ADHES) {
-                ox -= px;
-                oy -= py;
-                as_global(I.poldx)[ii] = ox;
-                as_global(I.poldy)[ii] = oy;
-            }
-            c0 = ox * ox + oy * oy;
+            ox = as_global(I.poldx)[ii];
+            oy = as_global(I.poldy)[ii];
         }
-        c1 = px * px + py * py;
-        if (s >= ADHES) c2 = rx * rx + ry * ry;
+        double dscl = as_global(I.dscl)[ii];
+        // the run of adhesion that this element ends: its first element is the nearest one, at or
+        // before this one, that begins the row or follows an element not in adhesion
+        auto begins = [&](int j) { return j % mx == 0 || as_global(I.el)[j - 1] != ADHES; };
+        const int lane = threadIdx.x & 63, w0 = i - lane;
+        const unsigned long long stop = __builtin_amdgcn_ballot_w64(!in || begins(i));
+        const unsigned long long mine = stop & (~0ull >> (63 - lane));
+        int start = w0 + 63 - __clzll((long long)mine);
+        if (!(stop & 1)) {
+            int prev = 0;
+            for (int c = w0 - 64; c >= 0; c -= 64) {
+                const unsigned long long b = __builtin_amdgcn_ballot_w64(begins(c + lane));
+                if (b) {
+                    prev = c + 63 - __clzll((long long)b);
+                    break;
+                }
+            }
+            if (!mine) start = prev;
+        }
+        double rx = 0.0, ry = 0.0, c0 = 0.0, c1 = 0.0, c2 = 0.0;
+        if (in) {
+            int8_t elnew = EXTER;
+            double fac_s = 0.0;
+            bool have = false;
+            if (s == SLIP) have = gd_slip_split(I, px, py, pn, sx, sy, elnew, fac_s);
+            if (s == SLIP && !have) {
+                // the reference keeps elnew/fac_s of the last slip element it split
+                for (int j = i - 1; j >= 0; j--) {
+                    if (I.el[j] != SLIP) continue;
+                    if (gd_slip_split(I, I.px[j], I.py[j], I.pn[j], I.sx[j], I.sy[j], elnew, fac_s)) break;
+                }
+            }
+            if (s == SLIP && elnew == SLIP) {
+                dscl = I.d_slp * pow(fac_s, I.pow_s);
+            } else if (s == ADHES || (s == SLIP && elnew == ADHES)) {
+                const int run = i - start;
+                double dnew;
+                if (I.d_cns < I.d_ifc)
+                    dnew = fmax(I.d_cns, I.d_ifc + (run - 1) * fmin(0.0, I.d_lin));
+                else
+                    dnew = fmin(I.d_cns, I.d_ifc + (run - 1) * fmax(0.0, I.d_lin));
+                dscl = fmin(50.0 * dscl, dnew);
+            } else if (s != ADHES) {
+                dscl = 0.0;
+            }
+            as_global(I.dscl)[ii] = dscl;
+            if (s == ADHES) {
+                rx = -sx * dscl;
+                ry = -sy * dscl;
+            } else if (s == SLIP) {
+                double tx = -ny, ty = nx;
+                double st = tx * sx + ty * sy;
+                rx = -st * tx * dscl;
+                ry = -st * ty * dscl;
+            }
+            as_global(I.rx)[ii] = rx;
+            as_global(I.ry)[ii] = ry;
+            if (!I.first) {
+                if (s >= ADHES) {
+                    ox -= px;
+                    oy -= py;
+                    as_global(I.poldx)[ii] = ox;
+                    as_global(I.poldy)[ii] = oy;
+                }
+                c0 = ox * ox + oy * oy;
+            }
+            c1 = px * px + py * py;
+            if (s >= ADHES) c2 = rx * rx + ry * ry;
+        }
+        con[0][own] = c0;
+        con[1][own] = c1;
+        con[2][own] = c2;
     }
-    con[0][threadIdx.x] = c0;
-    con[1][threadIdx.x] = c1;
-    con[2][threadIdx.x] = c2;
     __syncthreads();
     double acc[3] = {0.0, 0.0, 0.0};
     if (threadIdx.x < ELEM_THREADS)
@@ -4669,8 +4677,11 @@ void launch_op(int kind, const void* d_items, const int* d_gstart, int nitems, i
         if (ngroups <= N_CU) hipLaunchKernelGGL(k_gd_update<1024>, ge, dim3(1024), lds_bytes, s, (const GdItem*)d_items, d_gstart, nitems, ro);
         else hipLaunchKernelGGL(k_gd_update<256>, ge, dim3(256), lds_bytes, s, (const GdItem*)d_items, d_gstart, nitems, ro);
         break;
-    case OP_GD_MOVES: hipLaunchKernelGGL(k_gd_moves, ge, dim3(GD_ELEM_THREADS), 0, s, (const GdItem*)d_items, d_gstart, nitems, ro); break;
-    case OP_GD_DIAGRES: hipLaunchKernelGGL(k_gd_diagres, ge, dim3(GD_ELEM_THREADS), 0, s, (const GdItem*)d_items, d_gstart, nitems, ro); break;
+    case OP_GD_MOVES: hipLaunchKernelGGL(k_gd_moves, ge, dim3(GD_ELEM_TILE), 0, s, (const GdItem*)d_items, d_gstart, nitems, ro); break;
+    case OP_GD_DIAGRES:
+        if (ngroups <= N_CU) hipLaunchKernelGGL(k_gd_diagres<1024>, ge, dim3(1024), 0, s, (const GdItem*)d_items, d_gstart, nitems, ro);
+        else hipLaunchKernelGGL(k_gd_diagres<256>, ge, dim3(256), 0, s, (const GdItem*)d_items, d_gstart, nitems, ro);
+        break;
     case OP_SETUP: hipLaunchKernelGGL(k_setup, ge, te, 0, s, (const SetupItem*)d_items, d_gstart, nitems, ro); break;
     case OP_FORCES: hipLaunchKernelGGL(k_forces, ge, te, 0, s, (const SetupItem*)d_items, d_gstart, nitems, ro); break;
     case OP_STDYGS:

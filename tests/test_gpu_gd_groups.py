@@ -52,3 +52,21 @@ def test_long_adhesion(cntc, oracle, mx, my):
     assert (el == 1).sum(1).max() > 64
     for a, b in zip(p, P.tractions()):
         assert np.abs(a - b).max() <= 1e-8 * np.abs(P.tractions()[0]).max()
+
+
+def test_long_adhesion_in_many_groups(cntc):
+    """Runs of adhesion over several wavefronts where the scaling takes four elements a thread in turn."""
+    c = case(150, 9, 1e-6)
+    n, one = 140, 600    # two groups each
+    for k in range(n + 1):
+        W.apply_case(cntc, one + k, 1, c)
+    assert cntc.calculate(one, 1) == 0
+    err = cntc.calculatebatch(list(range(one + 1, one + n + 1)), [1] * n)
+    want = [a.tobytes() for a in cntc.gettractions(one, 1)]
+    its = cntc.getiterations(one, 1)
+    el = cntc.getelementdivision(one, 1).reshape(9, 150)
+    got = [([a.tobytes() for a in cntc.gettractions(one + k, 1)], cntc.getiterations(one + k, 1)) for k in range(1, n + 1)]
+    for k in range(n + 1):
+        cntc.finalize(one + k)
+    assert its[3] > 5 and not np.any(err) and (el == 1).sum(1).max() > 64
+    assert all(g[0] == want and g[1][:4] == its[:4] for g in got)
