@@ -1569,10 +1569,10 @@ __device__ void elmtrc(int8_t& el, const double c11, const double c12, const dou
 }
 
 // element-state moves after a GD step (src/gdsteady.f90:375-418); returns #changes.  An element
-// per thread: latency-bound by the slip elements' 2x2 problem.  Only the signs and states that
-// follow from its solution are used, so it is solved on the latency path (elmtrc, scale_dir).
-// With four elements in turn and the general problem 20.3 us a launch for a mix of sides 20 to 256,
-// 10.1 us so; 1024 x 1024 33.2 and 26.5 us (HIP events, about 4 us of each their own).
+// per thread: latency-bound by the slip elements' 2x2 problem, whose solution decides the state, so
+// with full divisions and angles.  Four elements in turn / one a thread: 40 x 40 17.7 and 10.5 us a
+// launch, 48 patches of sides 20 to 72 26.3 and 13.6, 1024 x 1024 55.1 and 36.3 (HIP events, about 4
+// us of each their own).
 __global__ void __launch_bounds__(GD_ELEM_TILE) k_gd_moves(const GdItem* __restrict__ items, const int* __restrict__ gstart,
                                                               int nitems, RedOut ro)
 {
@@ -1597,7 +1597,7 @@ __global__ void __launch_bounds__(GD_ELEM_TILE) k_gd_moves(const GdItem* __restr
         } else if (s == SLIP) {
             const double snrm = nx * si[0] + ny * si[1];
             int8_t elopt = s;
-            elmtrc(elopt, I.c11, I.c12, I.c21, I.c22, 1e-6, pr, I.mu, si, 1.0, 1.0, true);
+            elmtrc(elopt, I.c11, I.c12, I.c21, I.c22, 1e-6, pr, I.mu, si);
             double cosdth = (nx * pr[0] + ny * pr[1]) / g;
             if ((snrm > 0.0 && (dscl >= 0.001 || elopt == ADHES)) || cosdth <= -0.5) {
                 as_global(I.el)[ii] = ADHES;
