@@ -592,7 +592,7 @@ private:
         if (op.timed) HIPCHK(hipEventRecord(op.t0, op.stream));
         // one work-group per item: its partials are the item's results
         launch_op(kind, op.dev, (const int*)(op.dev + items_b), nitems, tot,
-                  RedOut{(double*)(op.dev + op.res_off), nullptr, nullptr, nullptr}, variant, lds, op.stream);
+                  RedOut{(double*)(op.dev + op.res_off), nullptr, nullptr}, variant, lds, op.stream);
         HIPCHK(hipGetLastError());
         if (op.timed) HIPCHK(hipEventRecord(op.t1, op.stream));
         HIPCHK(hipMemcpyAsync(op.host + op.res_off, op.dev + op.res_off, res_b, hipMemcpyDeviceToHost,
@@ -698,7 +698,7 @@ private:
         HIPCHK(hipStreamWaitEvent(op.stream, op.ev_start, 0));
         HIPCHK(hipMemcpyAsync(op.dev, op.host, items_b + gs_b, hipMemcpyHostToDevice, op.stream));
         launch_op(OP_GSB_SETUP, op.dev, (const int*)(op.dev + items_b), nitems, nitems,
-                  RedOut{(double*)(op.dev + op.res_off), nullptr, nullptr, nullptr}, 0, 0, op.stream);
+                  RedOut{(double*)(op.dev + op.res_off), nullptr, nullptr}, 0, 0, op.stream);
         HIPCHK(hipGetLastError());
         HIPCHK(hipMemcpyAsync(op.host + op.res_off, op.dev + op.res_off, res_b, hipMemcpyDeviceToHost,
                               op.stream));
@@ -944,7 +944,7 @@ private:
         // stage items, group tables and result slots
         struct Launch {
             int kind, nitems, K, stage;
-            size_t items_off, gstart_off, modes_off, part_off, res_off, cnt_off;
+            size_t items_off, gstart_off, part_off, res_off, cnt_off;
             int ngroups;
             size_t lds;
         };
@@ -999,10 +999,6 @@ private:
                     off = align(off + sizeof(int) * (nitems + 1));
                     L.ngroups = tot;
                     L.lds = lds;
-                    L.modes_off = off;
-                    int* md = (int*)(hstage_ + off);
-                    for (int i = 0; i < nitems; i++) md[i] = op_combine_mode(kind, &flat[g.reqs[i]]->item);
-                    off = align(off + sizeof(int) * nitems);
                     L.part_off = part;
                     L.res_off = res;
                     L.cnt_off = cnt;
@@ -1061,11 +1057,10 @@ private:
                 pkeys.push_back({L.kind * 4 + L.stage, bytes});
                 HIPCHK(hipEventRecord(ev_pool[nev++], s_));
             }
-            RedOut ro{dpart_ + L.part_off, L.K > 0 ? dcnt_ + L.cnt_off : nullptr, dres_ + L.res_off,
-                      (const int*)(dstage_ + L.modes_off)};
+            RedOut ro{dpart_ + L.part_off, L.K > 0 ? dcnt_ + L.cnt_off : nullptr, dres_ + L.res_off};
             // SteadyGS and ConvexGS write their one group's values as the item's results
             if (L.kind == OP_STDYGS || L.kind == OP_CNVXGS)
-                ro = RedOut{dres_ + L.res_off, nullptr, nullptr, nullptr};
+                ro = RedOut{dres_ + L.res_off, nullptr, nullptr};
             launch_op(L.kind, dstage_ + L.items_off, (const int*)(dstage_ + L.gstart_off), L.nitems,
                       L.ngroups, ro, L.stage, L.lds, s_);
             if (hipError_t le = hipGetLastError(); le != hipSuccess) {

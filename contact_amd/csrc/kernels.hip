@@ -4559,17 +4559,6 @@ int op_nred(int kind, const void* item)
     (void)item;
 }
 
-int op_combine_mode(int kind, const void* item)
-{
-    if (kind == OP_VEC) {
-        int sub = ((const VecItem*)item)->sub;
-        if (sub == V_MAXABS || sub == V_MAX) return 1;
-        if (sub == V_MIN) return 2;
-    }
-    if (kind == OP_SETUP || kind == OP_SENS_EXT) return 1;
-    return 0;
-}
-
 int op_groups(int kind, const void* item, int conv_stage)
 {
     switch (kind) {

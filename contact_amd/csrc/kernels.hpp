@@ -14,8 +14,6 @@ constexpr size_t MAX_LDS = 160 * 1024;
 
 // number of reduction values an item of `kind` produces (0: none)
 int op_nred(int kind, const void* item);
-// combine mode of the reduction: 0 sum, 1 max, 2 min
-int op_combine_mode(int kind, const void* item);
 // work-groups an item needs (conv_stage 0/1/2 selects the stage of an FFT product)
 int op_groups(int kind, const void* item, int conv_stage);
 // algorithmic HBM bytes of one item in one stage (for the bandwidth report)

@@ -13,12 +13,11 @@ namespace cntc {
 
 // Where a launch's reductions go: group partials [group * K + k]; with `count` set (one
 // counter per item, zero between launches) the last group of each item also combines them
-// into results [item * K + k] with the item's combine mode (modes[item]: 0 sum, 1 max, 2 min).
+// into results [item * K + k], as the operation combines its values (sum, max or min).
 struct RedOut {
     double* partials;
     unsigned* count;
     double* results;
-    const int* modes;
 };
 
 // element-state codes, src/m_gridfunc.f90:30-37
