@@ -1,5 +1,5 @@
 """SteadyGS by blocks of rows: interior rows just over 64, 128 and 256 elements (slots of the
-walk's registers), grids that fit 8, 5 and 1 rows per block, last blocks of few rows, and both the
+walk's registers), grids that take 8 and 5 rows per block, last blocks of few rows, and both the
 default and a fixed relaxation.
 
 Tolerance: the same sweeps as the oracle's up to rounding, stopped at eps 1e-9 of the traction's
@@ -30,8 +30,12 @@ def test_row_widths(cntc, oracle, mx, my, gausei):
     cntc.finalize(ire)
     rc, of, P = oracle.solve_case(c)
     assert rc == 0
-    print(mx, my, "widest row", (el > 0).sum(1).max(), "adhesion", (el == 1).sum(), "iterations", its, P.iters())
+    print(mx, my, "widest row", (el > 0).sum(1).max(), "adhesion", (el == 1).sum(), "iterations", its, P.iters(),
+          "clips", P.gs_clips())
     assert its[4] & 2, "SteadyGS did not run"
+    assert (el > 0).sum(1).max() > {9: 0, 69: 64, 134: 128, 262: 256, 450: 384}[mx]
+    # adhesion elements that a move takes over their bound, on the way or to the end
+    assert P.gs_clips() > 0
     for a, b in zip(p, P.tractions()):
         assert np.abs(a - b).max() <= 1e-7 * np.abs(P.tractions()[0]).max()
     for a, b in zip(f[:3], of[:3]):
