@@ -537,8 +537,11 @@ private:
             if (k >= order.size()) break;
             if (!side_idle(st)) continue;
             const long top = order[k]->item.gs.n;
+            const int form = gsb_walk_form(order[k]->item.gs.mx);
             std::vector<Req*> byvar[4];
-            for (size_t c = 0; k < order.size() && c < 64 && 4L * order[k]->item.gs.n >= top; k++, c++) {
+            for (size_t c = 0; k < order.size() && c < 64 && 4L * order[k]->item.gs.n >= top &&
+                               gsb_walk_form(order[k]->item.gs.mx) == form;
+                 k++, c++) {
                 Req* r = order[k];
                 int v = maxvar;
                 // (2 KB left for the kernels' static LDS)
@@ -885,7 +888,9 @@ private:
                     }
                     HIPCHK(hipEventRecord(G.wev[G.nwev], op.stream));
                 }
-                launch_op(L.kind, d + L.items, (const int*)(d + L.gst[0]), L.n, L.ng[0], ro, 0, L.lds[0],
+                // (the patches of a group take the same form of the walk)
+                const int form = L.kind == OP_GSB_WALK ? gsb_walk_form(G.gs[0].mx) : 0;
+                launch_op(L.kind, d + L.items, (const int*)(d + L.gst[0]), L.n, L.ng[0], ro, form, L.lds[0],
                           op.stream);
                 if (tw) {
                     HIPCHK(hipEventRecord(G.wev[G.nwev + 1], op.stream));

@@ -3648,7 +3648,7 @@ __host__ __device__ inline size_t gsb_lds(int mx, int rows, bool wide)
     const size_t cells = wide ? 24 : 24 + 6 * (rows - 1) + (rows > 1 ? 2 * rows + 12 : 0);
     return cells * mx * sizeof(double) + (size_t)4 * rows * sizeof(int) + 64;
 }
-constexpr int GSB_MAX_ROWS = 8, GSB_LDS_ROWS = 4;
+constexpr int GSB_MAX_ROWS = 8, GSB_LDS_ROWS = 5;
 // as many rows as fit the LDS beside the kernel's static part (0: not even one)
 __host__ __device__ inline int gsb_fit(int mx, bool wide)
 {
@@ -3657,11 +3657,12 @@ __host__ __device__ inline int gsb_fit(int mx, bool wide)
     return r;
 }
 // Each block of a sweep costs a product of the whole grid, so that blocks of few rows are dear.  The
-// LDS holds the coefficients of eight rows up to 214 columns, of four up to 325 and of one from 440
-// on; blocks of wider rows keep eight by reading them from memory.  Calls of some forty sweeps on 300
-// rows take, with 300 columns, 2.71 s from the LDS (four rows) and 2.80 from memory; 325: 3.07 (four)
-// and 3.05; 350: 6.8 (three) and 4.2; 450: 16.8 (one) and 7.9; 520: 25.6 (one) and 12.4 s.  On 24 rows
-// of 520 columns 0.63 and 0.31.
+// LDS holds the coefficients of eight rows up to 214 columns, of five up to 288, of four up to 325 and
+// of one from 440 on; blocks of wider rows keep eight by reading them from memory.  Calls of some forty
+// sweeps on 300 rows take, with 250 columns, 1.82 s from the LDS (six rows) and 1.92 from memory; 300:
+// 2.71 (four) and 2.80; 325: 3.07 (four) and 3.05; 350: 6.8 (three) and 4.2; 450: 16.8 (one) and 7.9;
+// 520: 25.6 (one) and 12.4 s.  On 24 rows of 520 columns 0.63 and 0.31.  The line is at five rows, where
+// the rows still fit five slots and with them 256 registers (see k_gsb_walk).
 __host__ __device__ inline bool gsb_wide(int mx) { return gsb_fit(mx, false) < GSB_LDS_ROWS; }
 __host__ __device__ inline int gsb_fit_rows(int mx) { return gsb_fit(mx, gsb_wide(mx)); }
 
@@ -4081,7 +4082,7 @@ __device__ __forceinline__ void gsb_walk_block(const GsbItem& I, double* const l
                 gsb_walk_row<ns>(row, ev, pt, mx, t0, t1, tab0, difacc, I.eps, I.omegah, I.omegas);
             };
             // slots of 64 elements, few of them beyond the row's end (each costs every element some
-            // 50 cycles); of the rows that the LDS form takes none has more than 325 elements
+            // 50 cycles); the LDS form takes rows of up to 288 elements
             if constexpr (WIDE) {
                 if (nt <= 256) walk(Count<4>());
                 else if (nt <= 384) walk(Count<6>());
@@ -4092,7 +4093,7 @@ __device__ __forceinline__ void gsb_walk_block(const GsbItem& I, double* const l
                 if (nt <= 64) walk(Count<1>());
                 else if (nt <= 128) walk(Count<2>());
                 else if (nt <= 256) walk(Count<4>());
-                else walk(Count<6>());
+                else walk(Count<5>());
             }
             flops += 4.0 * nt * nt;
         } else if (n < B) {
@@ -4203,14 +4204,15 @@ __device__ __forceinline__ void gsb_walk_block(const GsbItem& I, double* const l
     }
 }
 
-__global__ void __launch_bounds__(GSB_THREADS) k_gsb_walk(const GsbItem* __restrict__ items, const int* __restrict__ gstart,
-                                                          int nitems, RedOut ro)
+// Kernels of their own: 14 slots take nearly all registers of a compute unit's SIMDs, which is then the
+// walk's alone; with 256 of them the other patches' kernels run beside it (768 patches of sides 20 to
+// 256 at once, all in the LDS form: 70 patches/s with one kernel of 482 registers, 71.7 so).
+template <bool WIDE>
+__global__ void __launch_bounds__(GSB_THREADS, WIDE ? 1 : 2) k_gsb_walk(const GsbItem* __restrict__ items,
+                                                                        const int* __restrict__ gstart, int nitems)
 {
     extern __shared__ double gsb_lds_[];
-    (void)ro;
-    const GsbItem& I = items[find_item(gstart, nitems, blockIdx.x)];
-    if (gsb_wide(I.mx)) gsb_walk_block<true>(I, gsb_lds_);
-    else gsb_walk_block<false>(I, gsb_lds_);
+    gsb_walk_block<WIDE>(items[find_item(gstart, nitems, blockIdx.x)], gsb_lds_);
 }
 
 // end of a sweep (src/m_solvpt.f90:3130-3150): dif = sqrt(sum |dp|^2 / 2k), difid from the rms
@@ -4654,7 +4656,10 @@ void launch_op(int kind, const void* d_items, const int* d_gstart, int nitems, i
     case OP_CNVXGS: hipLaunchKernelGGL(k_cnvxgs, ge, dim3(64), 0, s, (const CgsItem*)d_items, d_gstart, nitems, ro); break;
     case OP_DENSE: hipLaunchKernelGGL(k_dense, ge, dim3(64 * DENSE_WAVES), 0, s, (const DenseItem*)d_items, d_gstart, nitems); break;
     case OP_GSB_SETUP: hipLaunchKernelGGL(k_gsb_setup, ge, dim3(GSB_THREADS), 0, s, (const GsbItem*)d_items, d_gstart, nitems, ro); break;
-    case OP_GSB_WALK: hipLaunchKernelGGL(k_gsb_walk, ge, dim3(GSB_THREADS), lds_bytes, s, (const GsbItem*)d_items, d_gstart, nitems, ro); break;
+    case OP_GSB_WALK:
+        if (conv_stage == 1) hipLaunchKernelGGL(k_gsb_walk<true>, ge, dim3(GSB_THREADS), lds_bytes, s, (const GsbItem*)d_items, d_gstart, nitems);
+        else hipLaunchKernelGGL(k_gsb_walk<false>, ge, dim3(GSB_THREADS), lds_bytes, s, (const GsbItem*)d_items, d_gstart, nitems);
+        break;
     case OP_GSB_CHECK: hipLaunchKernelGGL(k_gsb_check, ge, dim3(GSB_THREADS), 0, s, (const GsbItem*)d_items, d_gstart, nitems, ro); break;
     case OP_GD_PROJECT: hipLaunchKernelGGL(k_gd_project, ge, dim3(GD_ROW_THREADS), lds_bytes, s, (const GdItem*)d_items, d_gstart, nitems, ro); break;
     // with a CU to each group the most threads it can have; else those of which two groups share one
@@ -4820,6 +4825,7 @@ void launch_fill_u32(unsigned* p, size_t n, unsigned v, hipStream_t s)
 }
 
 int gsb_block_rows(int mx) { return gsb_fit_rows(mx); }
+int gsb_walk_form(int mx) { return gsb_wide(mx) ? 1 : 0; }
 
 void conv_default_shape(const ConvItem* c, int* rpg, int* cpg)
 {

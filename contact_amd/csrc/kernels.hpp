@@ -28,6 +28,9 @@ void launch_op(int kind, const void* d_items, const int* d_gstart, int nitems, i
 
 // rows per block of the block SteadyGS on grids of mx columns (0: not even one fits the LDS)
 int gsb_block_rows(int mx);
+// the walk kernel of such grids (conv_stage of OP_GSB_WALK, the same for all items of a launch): 0
+// with the block's coefficients in the LDS, 1 with them in memory
+int gsb_walk_form(int mx);
 // the default tile shapes of a product item (rows per work-group of the row stages, columns
 // per work-group of the column stage)
 void conv_default_shape(const ConvItem* c, int* rpg, int* cpg);

@@ -42,10 +42,11 @@ def test_row_widths(cntc, oracle, mx, my, gausei):
         assert abs(a - b) <= 1e-7 * c["fstat"] * c["fn"]
 
 
-# mx, my, elements that the widest row has to exceed: coefficients in the LDS for blocks of 7, 5 and 4
-# rows; read from memory for rows that take 6, 8, 11 and 14 slots, in blocks of 8 rows with a second
-# one of 5, 1 and none, and of 4 on the widest grid that blocks take
-WIDE = [(220, 12, 128), (288, 10, 256), (325, 9, 256), (326, 13, 256), (420, 9, 384), (560, 8, 512), (842, 8, 704)]
+# mx, my, elements that the widest row has to exceed: coefficients in the LDS for blocks of 7, 6 and 5
+# rows, of 4 and 5 slots; read from memory for rows that take 6, 8, 11 and 14 slots, in blocks of 8 rows
+# with a second one of 1, 5, 1 and none, and of 4 on the widest grid that blocks take
+WIDE = [(220, 12, 128), (250, 8, 192), (288, 10, 256), (325, 9, 256), (326, 13, 256), (420, 9, 384), (560, 8, 512),
+        (842, 8, 704)]
 
 
 @pytest.mark.parametrize("mx,my,wider", WIDE)
@@ -73,3 +74,26 @@ def test_wide_rows(cntc, oracle, mx, my, wider):
         assert np.abs(a - b).max() <= 1e-5 * np.abs(P.tractions()[0]).max()
     for a, b in zip(f[:3], of[:3]):
         assert abs(a - b) <= 1e-5 * c["fstat"] * c["fn"]
+
+
+def test_narrow_and_wide_grids_in_one_batch(cntc):
+    """Patches of both forms of the walk that wait together: the same bits as each alone."""
+    grids = [(30, 20), (300, 8), (60, 44), (500, 7), (100, 26), (289, 9), (288, 9), (842, 5), (25, 11)]
+    cases = [W.base_case(tang=3, norm=1, fn=9e4 * min(1.0, my / mx), cksi=-3e-4, ceta=1e-4, cphi=1e-4, eps=1e-4, ipotcn=-3,
+                         mx=mx, my=my, aa=6.0, bb=6.0 * min(1.0, my / mx), scale=max(mx / (mx - 4.0), 1.0), gausei=0)
+             for mx, my in grids]
+    ids = [(944, 1 + k) for k in range(len(grids))]
+    want = []
+    for (ire, icp), c in zip(ids, cases):
+        W.apply_case(cntc, ire, icp, c)
+        assert cntc.calculate(ire, icp) == 0
+        assert cntc.getiterations(ire, icp)[4] & 2, "SteadyGS did not run"
+        want.append([a.tobytes() for a in cntc.gettractions(ire, icp)])
+    cntc.finalize(944)
+    for (ire, icp), c in zip(ids, cases):
+        W.apply_case(cntc, ire, icp, c)
+    err = cntc.calculatebatch([i for i, _ in ids], [j for _, j in ids])
+    got = [[a.tobytes() for a in cntc.gettractions(*i)] for i in ids]
+    cntc.finalize(944)
+    assert not np.any(err)
+    assert got == want

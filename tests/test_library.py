@@ -39,7 +39,7 @@ def test_steadygs_rows_per_block(cntc):
     """SteadyGS by blocks: a product of the whole grid per block, so no block of a few rows, as far as
     the widest grid whose rows fit the LDS."""
     rows = getattr(ctypes.CDLL(cntc.library_path), "_ZN4cntc14gsb_block_rowsEi")
-    assert [rows(mx) for mx in (11, 214, 215, 325, 326, 440, 668, 841)] == [8, 8, 7, 4, 8, 8, 8, 8]
+    assert [rows(mx) for mx in (11, 214, 215, 288, 289, 440, 668, 841)] == [8, 8, 7, 5, 8, 8, 8, 8]
     assert all(rows(mx) >= 4 for mx in range(2, 843)) and rows(843) == 0
 
 
