@@ -144,7 +144,10 @@ __device__ inline double combine_identity(int mode)
 // needs no arrival at all.  With several groups, only the partials pass between groups: they
 // are stored and loaded as agent-scope atomics (past the caches of the XCD), and the group waits
 // for its stores before it arrives.  A fence would first write the XCD's L2 back, the vectors
-// that the kernel has just stored included.  Measured (k_vec, average over its operations of a
+// that the kernel has just stored included.  The order rests on gfx950's instructions, not on the
+// language's memory model, which asks for a release and an acquire: agent-scope stores are written
+// through to where every XCD's agent-scope loads look, s_waitcnt vmcnt(0) ends once they are there, and
+// one wavefront stores, waits, arrives and, as the last, loads.  Measured (k_vec, average over its operations of a
 // solve, HIP events of about 4 us included): 42.0 us a launch with fences and LDS shuffles, 18.4
 // us so for one 1024 x 1024 patch (1024 groups), 18.9 and 9.8 us for 512 x 512, 12.5 and 7.1 us
 // for 40 x 40.
@@ -877,9 +880,10 @@ __device__ inline int8_t gd_state(const GdBound& b)
 // branch 30).  The cells are read from LDS four ahead of their use; a step in which every row
 // of the wave is in the exterior or below its bound ends after one comparison; there is no
 // other branch in the usual range.
-//   p g / |p|: the square root is the correctly rounded one (two corrections of the hardware
-// estimate); the half reciprocal left over from it needs one correction to start the two
-// divisions, and each ends with the residual correction that rounds it correctly: the bits of
+//   p g / |p|: Goldschmidt's iteration for the square root and its half reciprocal from the hardware
+// estimate, with Markstein's residual corrections at the end: the square root is the correctly rounded
+// one; the half reciprocal needs one more correction to start the two divisions, and each ends with the
+// residual correction that rounds it correctly: the bits of
 // px * g / sqrt(px * px + py * py) without the range handling of the general sequences, which
 // serve the steps where |p|^2 leaves 2^+-600.  A step in slip takes about 300 cycles so, with the
 // compiler's square root and divisions and the reads in place 580 (k_gd_probe of one 512 x 512
@@ -1149,8 +1153,9 @@ __global__ void __launch_bounds__(GD_ROW_THREADS, 4) k_gd_project(const GdItem* 
 // Latency-bound: the row chain, then atan2, cos and sin per element.  The terms take all T
 // threads; each element's are left in its LDS cells and added up by 256 of the threads, element
 // t, t + 256, ... each, so that the sums do not depend on T.  With 256 threads for
-// all of it, eight elements in turn each: 26.4 us a launch for a mix of sides 20 to 256, 25.2 us
-// so; 512 x 512 88.9 and 88.2 us (HIP events, about 4 us of each their own).
+// all of it, eight elements in turn each: 40 x 40 22.2 us a launch, 19.1 us so; 48 patches of sides 20
+// to 72 27.5 and 23.9; 512 x 512 95.2 and 91.1; 1024 x 1024 (512 threads) 145.2 and 140.5 us (HIP
+// events, about 4 us of each their own).
 template <int T>
 __global__ void __launch_bounds__(T, 4) k_gd_probe(const GdItem* __restrict__ items, const int* __restrict__ gstart,
                                                    int nitems, RedOut ro)
@@ -3792,7 +3797,7 @@ __device__ inline void elmtrc_uniform(int& el, double c11, double c22, double ep
 //   - the next element's data and coefficients are read from LDS while this one is solved.
 //   - every lane solves the element on the same data (scalar branches, elmtrc_uniform).
 // An adhesion element upstream that the move takes over its bound is clipped and the elements
-// below it move by its change: one more term of u for each (rare).
+// below it move by its change: one more term of u for each (most of them in the first sweeps).
 // tab: own-row coefficients (xx, yy) times 1/G, offsets q - mx.
 template <int NS>
 __device__ __forceinline__ void gsb_walk_row(GsbEl* const row, const double* early, const double* part, int mx,
@@ -3962,7 +3967,7 @@ __device__ __forceinline__ void gsb_walk_row(GsbEl* const row, const double* ear
 // Latency-bound: one wavefront's chain.  With the sum over the row
 // formed for each element, and every row pair's coefficients staged from memory in the gap
 // between two rows, a block of eight rows of a 151 x 97 patch took 1515 us (2.1 us an element),
-// 589 us so; a sweep of an 11 x 11 patch 310 us, 52 us so.
+// 590 us so; a sweep of an 11 x 11 patch 310 us, 51 us so; of a 25 x 25 one 302 and 75 us.
 template <bool WIDE>
 __device__ __forceinline__ void gsb_walk_block(const GsbItem& I, double* const lds)
 {
